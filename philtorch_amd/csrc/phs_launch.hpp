@@ -217,9 +217,6 @@ int launch(int64_t B, int64_t T, bool TV, bool shared, bool backward, const void
     else
       a.partials = ws + L.partials_off;
   }
-  bool vec = (size_t(T) * sizeof(typename Alg::s_state)) % 16 == 0 && aligned16(x) && aligned16(y) &&
-             aligned16(out) && aligned16(a.gcoef) && (!TV || aligned16(coef));
-  a.vec_ok = vec ? 1 : 0;
 
   const void *kernel = TV ? (backward ? reinterpret_cast<const void *>(scan_kernel<Alg, true, true>)
                                        : reinterpret_cast<const void *>(scan_kernel<Alg, true, false>))

@@ -52,7 +52,6 @@ LpvSsArgs<Alg> lpv_args(int64_t B, int64_t T, const void *A, bool A_sh, bool A_t
   const unsigned sl = g_spin_limit.load(std::memory_order_relaxed);
   a.spin_limit = sl ? sl : kDefaultSpinLimit;
   a.agg_only = g_agg_only.load(std::memory_order_relaxed) ? 1u : 0u;
-  a.vec_ok = (size_t(T) * sizeof(E)) % 16 == 0 && aligned16(x) && aligned16(y) && aligned16(A);
   return a;
 }
 
@@ -85,8 +84,6 @@ int lpv_ss_fwd(int64_t B, int64_t T, const void *A, bool A_sh, bool A_tr, LpvOpe
   LpvSsArgs<Alg> a = lpv_args<Alg>(B, T, A, A_sh, A_tr, bv, cv, out_idx, 0, d, zi, x, y, zf, workspace);
   if (hs) {
     a.hs = static_cast<E *>(hs);
-    a.vec_hs = aligned16(hs) && (size_t(T) * sizeof(typename Alg::s_state)) % 16 == 0 && aligned16(x) &&
-               (size_t(T) * sizeof(E)) % 16 == 0;
     return rev ? lpv_launch<Alg, true, kSsStatesY>(a, stream) : lpv_launch<Alg, false, kSsStatesY>(a, stream);
   }
   return rev ? lpv_launch<Alg, true>(a, stream) : lpv_launch<Alg, false>(a, stream);
@@ -177,8 +174,6 @@ int lpv_ss_bwd(int64_t B, int64_t T, const void *A, bool A_sh, bool A_tr, LpvOpe
   if (T > 0) {
     LpvSsArgs<Alg> p = lpv_args<Alg>(B, T, A, A_sh, A_tr, bv, cv, out_idx, 0, d, zi, x, nullptr, nullptr, workspace);
     p.hs = states;
-    p.vec_hs = aligned16(states) && (size_t(T) * sizeof(SS)) % 16 == 0 && aligned16(x) &&
-               (size_t(T) * sizeof(E)) % 16 == 0;
     int rc = PHS_OK;
     if (!hs_in) {
       rc = rev ? lpv_launch<Alg, true, kSsStates>(p, stream) : lpv_launch<Alg, false, kSsStates>(p, stream);
@@ -188,7 +183,6 @@ int lpv_ss_bwd(int64_t B, int64_t T, const void *A, bool A_sh, bool A_tr, LpvOpe
     LpvSsArgs<Alg> q = lpv_args<Alg>(B, T, A, A_sh, !A_tr, cv, bv, 0, out_idx, d, gzf, gy, gx, gzi, workspace);
     q.hs_fwd = states;
     q.x_fwd = static_cast<const E *>(x);
-    q.vec_hs = p.vec_hs;
     q.gA_step = step_dst[0];
     q.gb_step = step_dst[1];
     q.gc_step = step_dst[2];

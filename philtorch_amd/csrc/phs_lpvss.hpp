@@ -59,7 +59,6 @@ struct LpvSsArgs {
   // they are constant in time ([B, tiles, kWaves, SsGrad::kN])
   E *hs;
   const E *hs_fwd, *x_fwd;
-  int vec_hs;
   E *gA_step, *gb_step, *gc_step, *gd_step;
   int gA_trans;
   int sum_b, sum_c, sum_d;
@@ -71,7 +70,6 @@ struct LpvSsArgs {
   unsigned tiles, per_stripe, spin_limit;
   unsigned agg_only;  // testing: tiles after a row's first publish no inclusive state
   uint64_t *status;
-  int vec_ok;
 };
 
 // 3 data waves and a look-back wave; the time-varying scan's steps per lane
@@ -93,11 +91,11 @@ struct LpvSsShape {
 // is time s; reversed (REV), time T-1-s, so the chunk is the K items below
 // T - s0 read in descending time.  Positions past the row read `fill`.
 template <bool REV, typename X, int K>
-__device__ __forceinline__ void lpv_load(const X *row, int64_t s0, int64_t T, bool vec, X (&out)[K], const X fill) {
+__device__ __forceinline__ void lpv_load(const X *row, int64_t s0, int64_t T, X (&out)[K], const X fill) {
   constexpr bool kVec = (K * sizeof(X)) % 16 == 0;
   if constexpr (!REV) {
     if constexpr (kVec) {
-      load_chunk<X, K>(row, s0, T, vec, out, fill);
+      load_chunk<X, K>(row, s0, T, out, fill);
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
@@ -109,9 +107,9 @@ __device__ __forceinline__ void lpv_load(const X *row, int64_t s0, int64_t T, bo
     }
   } else {
     const int64_t base = T - s0 - K;
-    if (kVec && vec && base >= 0) {
+    if (kVec && base >= 0) {
       X tmp[K];
-      if constexpr (kVec) load_chunk<X, K>(row, base, T, true, tmp, fill);
+      if constexpr (kVec) load_chunk<X, K>(row, base, T, tmp, fill);
 #pragma unroll
       for (int k = 0; k < K; ++k) out[k] = tmp[K - 1 - k];
     } else {
@@ -128,11 +126,11 @@ __device__ __forceinline__ void lpv_load(const X *row, int64_t s0, int64_t T, bo
 }
 
 template <bool REV, typename X, int K>
-__device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, bool vec, const X (&v)[K]) {
+__device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X (&v)[K]) {
   constexpr bool kVec = (K * sizeof(X)) % 16 == 0;
   if constexpr (!REV) {
     if constexpr (kVec) {
-      store_chunk<X, K>(row, s0, T, vec, v);
+      store_chunk<X, K>(row, s0, T, v);
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k)
@@ -140,11 +138,11 @@ __device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, bool ve
     }
   } else {
     const int64_t base = T - s0 - K;
-    if (kVec && vec && base >= 0) {
+    if (kVec && base >= 0) {
       X tmp[K];
 #pragma unroll
       for (int k = 0; k < K; ++k) tmp[k] = v[K - 1 - k];
-      if constexpr (kVec) store_chunk<X, K>(row, base, T, true, tmp);
+      if constexpr (kVec) store_chunk<X, K>(row, base, T, tmp);
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
@@ -257,8 +255,8 @@ __device__ __noinline__ typename Alg::state lpv_prefix_fallback(const LpvSsArgs<
     E u[K];
     SS xs[K];
     SC cs[K];
-    lpv_load<REV, E, K>(xrow, c0, a.T_len, a.vec_ok != 0, u, E(0));
-    lpv_load<REV, SC, K>(crow, c0, a.T_len, a.vec_ok != 0, cs, Alg::s_czero());
+    lpv_load<REV, E, K>(xrow, c0, a.T_len, u, E(0));
+    lpv_load<REV, SC, K>(crow, c0, a.T_len, cs, Alg::s_czero());
     if (a.A_trans) {
 #pragma unroll
       for (int k = 0; k < K; ++k) cs[k] = Alg::s_adjoint(cs[k]);  // real: the transpose
@@ -306,7 +304,6 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
   int64_t q, b;  // tile position along the row, row
   split_tile(id, a.B, a.b_magic, a.b_shift, q, b);
   const int64_t T = a.T_len;
-  const bool vec = a.vec_ok != 0;
   auto op = [](const M &p, const M &q2) { return compose<Alg>(p, q2); };
 
   if (w == kWaves) {
@@ -345,8 +342,8 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
   SC A[R][K];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    lpv_load<REV, E, K>(xrow, chunk0(r), T, vec, U[r], E(0));
-    lpv_load<REV, SC, K>(crow, chunk0(r), T, vec, A[r], Alg::s_czero());
+    lpv_load<REV, E, K>(xrow, chunk0(r), T, U[r], E(0));
+    lpv_load<REV, SC, K>(crow, chunk0(r), T, A[r], Alg::s_czero());
     if (a.A_trans) {
 #pragma unroll
       for (int k = 0; k < K; ++k) A[r][k] = Alg::s_adjoint(A[r][k]);  // real: the transpose
@@ -378,7 +375,6 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
   const E *cp = a.cv.p ? a.cv.p + b * a.cv.row_stride : nullptr;
   const E *dp = a.d.p ? a.d.p + b * a.d.row_stride : nullptr;
   const SS c_fixed = V::unit(a.out_idx);
-  const bool vh = a.vec_hs != 0;
   SsGrad<Alg, E> lacc;
   if constexpr (MODE == kSsGrad) {
 #pragma unroll
@@ -391,8 +387,8 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
     SS Hf[K];
     E Xf[K];
     if constexpr (MODE == kSsGrad) {
-      lpv_load<REV, SS, K>(reinterpret_cast<const SS *>(a.hs_fwd) + b * T, t0, T, vh, Hf, SS{});
-      lpv_load<REV, E, K>(a.x_fwd + b * T, t0, T, vh, Xf, E(0));
+      lpv_load<REV, SS, K>(reinterpret_cast<const SS *>(a.hs_fwd) + b * T, t0, T, Hf, SS{});
+      lpv_load<REV, E, K>(a.x_fwd + b * T, t0, T, Xf, E(0));
     }
     E O[K];
 #pragma unroll
@@ -417,11 +413,11 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
       }
     }
     if constexpr (MODE == kSsStates || MODE == kSsStatesY)
-      lpv_store<REV, SS, K>(reinterpret_cast<SS *>(a.hs) + b * T, t0, T, vh, Hf);
+      lpv_store<REV, SS, K>(reinterpret_cast<SS *>(a.hs) + b * T, t0, T, Hf);
     if constexpr (MODE == kSsPlain || MODE == kSsStatesY)
-      lpv_store<REV, E, K>(a.y + b * T, t0, T, vec, O);
+      lpv_store<REV, E, K>(a.y + b * T, t0, T, O);
     else if (MODE == kSsGrad && a.y)
-      lpv_store<REV, E, K>(a.y + b * T, t0, T, vec, O);
+      lpv_store<REV, E, K>(a.y + b * T, t0, T, O);
   }
   if constexpr (MODE == kSsGrad) {
     if (a.gpart) {  // the wave's sums of the operands constant in time

@@ -517,7 +517,6 @@ int lpv_mimo_ss(int F, int P, int64_t B, int64_t T, const void *A, int A_flags, 
   a.A = static_cast<const E *>(A);
   a.A_stride = (A_flags & PHS_LPV_A_SHARED) ? 0 : T * M * M;
   a.A_trans = (A_flags & PHS_LPV_A_TRANSPOSED) ? 1 : 0;
-  a.A_vec = aligned16(A) && (size_t(T) * M * M * sizeof(E)) % 16 == 0;
   a.Bm = static_cast<const E *>(Bm);
   a.b_stride = (shared & PHS_MIMO_B_SHARED) ? 0 : int64_t(M) * F;
   a.Cm = static_cast<const E *>(Cm);

@@ -40,7 +40,6 @@ struct MimoArgs {
   const E *A;  // [rows, M, M] row-major; time-varying (lpv_mimo_kernel): [rows, T, M, M]
   int64_t A_stride;  // elements between rows (0 = shared)
   int A_trans;       // time-varying: read each step's matrix transposed (the adjoint model's A[t]^T)
-  int A_vec;         // time-varying: a row's matrices lie in whole 16-byte vectors
   const E *Bm;  // [rows, M, F]
   int64_t b_stride;
   const E *Cm;  // [rows, P, M]
@@ -496,7 +495,7 @@ __device__ __forceinline__ void lpv_mimo_load_A(const MimoArgs<Alg> &a, int64_t 
                                                 typename Alg::s_coef (&Ak)[K]) {
   using SC = typename Alg::s_coef;
   const SC *row = reinterpret_cast<const SC *>(a.A + b * a.A_stride);
-  lpv_load<REV, SC, K>(row, s0, a.T_len, a.A_vec != 0, Ak, Alg::s_czero());
+  lpv_load<REV, SC, K>(row, s0, a.T_len, Ak, Alg::s_czero());
   if (a.A_trans) {
 #pragma unroll
     for (int k = 0; k < K; ++k) Ak[k] = Alg::s_adjoint(Ak[k]);  // real: the transpose

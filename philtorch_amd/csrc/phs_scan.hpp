@@ -128,7 +128,6 @@ struct ScanArgs {
   uint64_t b_magic;
   unsigned b_shift;
   uint64_t *status;          // status words of this call
-  int vec_ok;
   // tracing launches only (scan_kernel<..., TRACE = true>): per-tile phase
   // records, kTraceWords 64-bit words per tile id, for ids below trace_tiles
   uint64_t *trace;
@@ -247,6 +246,22 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// ------------------------------------------------------------ vectors of a row
+// Rows are read and written 16 bytes at a time wherever the 16 bytes lie
+// inside them, at any element alignment: a global memory instruction of four
+// words needs word alignment only, and torch and the C ABI give element
+// alignment (4 bytes at least).  A row of an odd number of fp32 steps starts
+// 4, 8 or 12 bytes past a 16-byte boundary in three rows of four.  Where such
+// rows took one element at a time (64 separate segments per instruction), 16
+// rows of 480001 steps against 480000 took (us, odd / even length before,
+// then odd now): order-2 lfilter 60.7 / 21.8, 21.6; filtfilt 119.6 / 40.5,
+// 40.3; complex64 lti_recur forward (64 rows) 231 / 128, 130; eight trained
+// sections 352 / 250, 253; 2x2 scan, forward and backward, 222 / 168, 169.
+struct __attribute__((packed, aligned(4))) RowVec {
+  uint32_t x, y, z, w;
+};
+__device__ __forceinline__ RowVec row_vec(const uint4 &v) { return {v.x, v.y, v.z, v.w}; }
+
 // ------------------------------------------------------------ coalesced stores
 // A lane that owns K consecutive steps writes them as NV 16-byte vectors of
 // its own, so one store instruction of the wave touches 64 separate
@@ -283,16 +298,17 @@ __device__ __forceinline__ void lds_put_chunk(uint4 *wb, int L, const X (&v)[K])
   for (int i = 0; i < NV; ++i) wb[L * NV + (i ^ sw)] = t.u[i];
 }
 
-// The wave's buffer to its block at dst (16-byte aligned, in range): vector
-// c of the block is block lane c / NV's vector c % NV.
+// The wave's buffer to its block at dst (in range): vector c of the block is
+// block lane c / NV's vector c % NV.
 template <int NV>
-__device__ __forceinline__ void lds_flush(uint4 *dst, const uint4 *wb, int lane, bool write) {
+__device__ __forceinline__ void lds_flush(void *dst, const uint4 *wb, int lane, bool write) {
   wave_sync();
   if (write) {
+    RowVec *out = static_cast<RowVec *>(dst);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int c = j * 64 + lane, L = c / NV, v = c % NV;
-      dst[c] = wb[L * NV + (v ^ lds_swizzle<NV>(L))];
+      out[c] = row_vec(wb[L * NV + (v ^ lds_swizzle<NV>(L))]);
     }
   }
   wave_sync();  // later writes to the buffer follow these reads
@@ -423,20 +439,19 @@ __device__ bool lookback(const uint64_t *row_status, const typename Alg::state &
 // The bounds-checked tail assigns in branches: `c ? row[t] : fill` with both
 // operands lvalues is an lvalue, compiled as a select between a global and a
 // private address, and every thread of the kernel then keeps a copy of
-// `fill` in scratch memory.  kFull: the caller knows the chunk is in range
-// and 16-byte aligned, so only the vector path is compiled (no branch
-// between the forms; see the kernel's full-tile path).
+// `fill` in scratch memory.  kFull: the caller knows the chunk is in range,
+// so only the vector path is compiled (no branch between the forms; see the
+// kernel's full-tile path).
 template <typename X, int K, bool kFull = false>
-__device__ __forceinline__ void load_chunk(const X *row, int64_t t0, int64_t T, bool vec, X (&out)[K],
-                                           const X fill) {
-  if (kFull || (vec && t0 + K <= T)) {
+__device__ __forceinline__ void load_chunk(const X *row, int64_t t0, int64_t T, X (&out)[K], const X fill) {
+  if (kFull || t0 + K <= T) {
     constexpr int nv = int(K * sizeof(X) / 16);
     static_assert(K * sizeof(X) % 16 == 0, "chunk must be 16-byte granular");
     union {
       X x[K];
-      uint4 v[nv];
+      RowVec v[nv];
     } u;
-    const uint4 *p = reinterpret_cast<const uint4 *>(row + t0);
+    const RowVec *p = reinterpret_cast<const RowVec *>(row + t0);
 #pragma unroll
     for (int i = 0; i < nv; ++i) u.v[i] = p[i];
 #pragma unroll
@@ -453,16 +468,16 @@ __device__ __forceinline__ void load_chunk(const X *row, int64_t t0, int64_t T, 
 }
 
 template <typename X, int K, bool kFull = false>
-__device__ __forceinline__ void store_chunk(X *row, int64_t t0, int64_t T, bool vec, const X (&v)[K]) {
-  if (kFull || (vec && t0 + K <= T)) {
+__device__ __forceinline__ void store_chunk(X *row, int64_t t0, int64_t T, const X (&v)[K]) {
+  if (kFull || t0 + K <= T) {
     constexpr int nv = int(K * sizeof(X) / 16);
     union {
       X x[K];
-      uint4 v[nv];
+      RowVec v[nv];
     } u;
 #pragma unroll
     for (int k = 0; k < K; ++k) u.x[k] = v[k];
-    uint4 *p = reinterpret_cast<uint4 *>(row + t0);
+    RowVec *p = reinterpret_cast<RowVec *>(row + t0);
 #pragma unroll
     for (int i = 0; i < nv; ++i) p[i] = u.v[i];
   } else {
@@ -513,8 +528,8 @@ __device__ __forceinline__ Map<Alg> lane_map(const typename Alg::s_coef (&Ac)[TV
 template <class Alg, bool TV, bool REV>
 __device__ __noinline__ typename Alg::state row_prefix_fallback(const typename Alg::s_state *xrow,
                                                                const typename Alg::s_coef *crow, int64_t T,
-                                                               bool vec, int64_t span, int64_t row_end,
-                                                               int lane, typename Alg::state virt) {
+                                                               int64_t span, int64_t row_end, int lane,
+                                                               typename Alg::state virt) {
   using SC = typename Alg::s_coef;
   using SS = typename Alg::s_state;
   using M = Map<Alg>;
@@ -528,8 +543,8 @@ __device__ __noinline__ typename Alg::state row_prefix_fallback(const typename A
     const int64_t c0 = REV ? row_end - off - int64_t(lane + 1) * K : off + int64_t(lane) * K;
     SS xs[K];
     SC cs[TV ? K : 1];
-    load_chunk<SS, K>(xrow, c0, T, vec, xs, zero_ss);
-    if constexpr (TV) load_chunk<SC, K>(crow, c0, T, vec, cs, zero_sc);
+    load_chunk<SS, K>(xrow, c0, T, xs, zero_ss);
+    if constexpr (TV) load_chunk<SC, K>(crow, c0, T, cs, zero_sc);
     M m = lane_map<Alg, TV, REV, K>(cs, xs, a_row_s);
     m = wave_scan_incl(m, lane, op);
     acc = compose<Alg>(acc, read_lane(m, 63));
@@ -575,7 +590,7 @@ __device__ __forceinline__ typename Alg::state tile_entry(const ScanArgs<Alg> &a
     if (!lookback<Alg>(row_status, virt, lane, tag, a.spin_limit, s_look, lb, yin))
       yin = row_prefix_fallback<Alg, TV, REV>(reinterpret_cast<const SS *>(a.x) + b * a.T_len,
                                               reinterpret_cast<const SC *>(a.coef) + b * a.coef_row_stride,
-                                              a.T_len, a.vec_ok != 0, qs * Sh::kTile, a.tiles_per_row * Sh::kTile,
+                                              a.T_len, qs * Sh::kTile, a.tiles_per_row * Sh::kTile,
                                               lane, virt);
   }
   if (qs + 1 < a.tiles_per_row && lane == 0 && !(a.agg_only && qs > 0))
@@ -600,7 +615,7 @@ __device__ __forceinline__ typename Alg::state tile_entry(const ScanArgs<Alg> &a
 // early writes mix into the co-resident tiles' reads (C1 backward 14.8 ->
 // 16.6 us, C5 fp64 step 1.80 -> 1.85 ms, same-box A/B).
 //
-// Full tiles (in range and 16-byte aligned) of real scalar scans and of
+// Full tiles (wholly inside the row) of real scalar scans and of
 // every backward run a copy of the data path with
 // only vector loads and stores, so the compiler's memory-counter waits see
 // one straight-line sequence of loads and each round's fold waits for its
@@ -702,7 +717,6 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
   split_tile(id, a.B, a.b_magic, a.b_shift, qs, b);
   const int64_t qf = REV ? a.tiles_per_row - 1 - qs : qs;  // position along time
   const int64_t T = a.T_len;
-  const bool vec = a.vec_ok != 0;
 
   const SS *xrow = reinterpret_cast<const SS *>(a.x) + b * T;
   const SC *crow = reinterpret_cast<const SC *>(a.coef) + b * a.coef_row_stride;
@@ -774,8 +788,7 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
   SC *gcrow = (REV && a.gcoef) ? reinterpret_cast<SC *>(a.gcoef) + b * T : nullptr;
 
   // The data path, compiled twice: kFull for tiles wholly inside the row
-  // with aligned rows (vector loads and stores only), and the bounds-checked
-  // form for the rest.
+  // (vector loads and stores only), and the bounds-checked form for the rest.
   auto data_path = [&](auto full_c) {
     constexpr bool kFull = decltype(full_c)::value;
     // ---- loads (all rounds issued up front)
@@ -786,10 +799,10 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int64_t t0 = chunk0(r);
-      load_chunk<SS, K, kFull>(xrow, t0, T, vec, X[r], zero_ss);
-      if constexpr (TV) load_chunk<SC, K, kFull>(crow, t0, T, vec, A[r], zero_sc);
+      load_chunk<SS, K, kFull>(xrow, t0, T, X[r], zero_ss);
+      if constexpr (TV) load_chunk<SC, K, kFull>(crow, t0, T, A[r], zero_sc);
       if constexpr (REV) {
-        load_chunk<SS, K, kFull>(yrow_in, t0, T, vec, Y[r], zero_ss);
+        load_chunk<SS, K, kFull>(yrow_in, t0, T, Y[r], zero_ss);
         Ylow[r] = zero_ss;
         if (lane == 63) {
           if (t0 == 0)
@@ -808,9 +821,9 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
     auto pass2 = [&](int r, SS h) -> AC {
       AC acc = Alg::acc_zero();
       const int64_t t0 = chunk0(r);
-      // the round's block (lowest time first) and whether it is whole and aligned
+      // the round's block (lowest time first) and whether it is whole
       const int64_t blk0 = t0 - int64_t(pl) * K;
-      const bool blk_full = kFull || (vec && blk0 + 64 * K <= T);
+      const bool blk_full = kFull || blk0 + 64 * K <= T;
       uint4 *wb = s_out + w * 64 * kNVb;
       if constexpr (!REV) {
         SS O[K];
@@ -822,10 +835,10 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
         if (kSLds && blk_full) {
           if constexpr (kSLds) {
             lds_put_chunk<SS, K>(wb, pl, O);
-            lds_flush<kNVs>(reinterpret_cast<uint4 *>(yrow + blk0), wb, lane, true);
+            lds_flush<kNVs>(yrow + blk0, wb, lane, true);
           }
         } else {
-          store_chunk<SS, K, kFull>(yrow, t0, T, vec, O);
+          store_chunk<SS, K, kFull>(yrow, t0, T, O);
         }
       } else {
         SS nu = h;
@@ -848,19 +861,19 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
         if (kSLds && blk_full) {
           if constexpr (kSLds) {
             lds_put_chunk<SS, K>(wb, pl, GX);
-            lds_flush<kNVs>(reinterpret_cast<uint4 *>(gxrow + blk0), wb, lane, gxrow != nullptr);
+            lds_flush<kNVs>(gxrow + blk0, wb, lane, gxrow != nullptr);
           }
         } else if (gxrow) {
-          store_chunk<SS, K, kFull>(gxrow, t0, T, vec, GX);
+          store_chunk<SS, K, kFull>(gxrow, t0, T, GX);
         }
         if constexpr (TV) {
           if (kCLds && blk_full) {
             if constexpr (kCLds) {
               lds_put_chunk<SC, K>(wb, pl, GC);
-              lds_flush<kNVc>(reinterpret_cast<uint4 *>(gcrow + blk0), wb, lane, gcrow != nullptr);
+              lds_flush<kNVc>(gcrow + blk0, wb, lane, gcrow != nullptr);
             }
           } else if (gcrow) {
-            store_chunk<SC, K, kFull>(gcrow, t0, T, vec, GC);
+            store_chunk<SC, K, kFull>(gcrow, t0, T, GC);
           }
         }
       }
@@ -945,7 +958,7 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
   // keep the single bounds-checked form: with the vector-only copy beside it
   // they measured slower (C2 forward 0.852 -> 0.861 ms, same-box A/B).
   constexpr bool kSplit = !Sh::kLookbackWave || REV;
-  if (kSplit && vec && (qf + 1) * Sh::kTile <= T)
+  if (kSplit && (qf + 1) * Sh::kTile <= T)
     data_path(std::true_type{});
   else
     data_path(std::false_type{});

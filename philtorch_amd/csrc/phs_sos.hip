@@ -157,7 +157,6 @@ int sos_fwd(int64_t B, int64_t T, int S, const SosCoefs &k, const void *zi, cons
   a.virt = static_cast<const E *>(zi);
   a.fin = static_cast<E *>(zf);
   a.ckpt = static_cast<Vec2<typename Wide<E>::type> *>(ckpt);
-  a.vec_ok = (size_t(T) * sizeof(E)) % 16 == 0 && aligned16(x) && aligned16(y);
   const unsigned grid = a.per_stripe * kStripes;
   launch_kernel((sos_kernel<E, Sh, false, false>), dim3(grid), dim3(Sh::kThreads), 0, stream, a);
   return hipGetLastError() == hipSuccess ? PHS_OK : PHS_ERR_LAUNCH;
@@ -188,7 +187,6 @@ int sos_bwd(int64_t B, int64_t T, int S, const SosCoefs &k, const void *x, const
   a.ckpt = const_cast<Vec2<typename Wide<E>::type> *>(static_cast<const Vec2<typename Wide<E>::type> *>(ckpt));
   a.x = static_cast<const E *>(x);
   a.partials = grad ? reinterpret_cast<typename Wide<E>::type *>(ws + L.partials_off) : nullptr;
-  a.vec_ok = (size_t(T) * sizeof(E)) % 16 == 0 && aligned16(gy) && aligned16(gx) && (!grad || aligned16(x));
   const unsigned grid = a.per_stripe * kStripes;
   if (grad) {
     // lane entry states of every section, then the kept sections' inputs:

@@ -102,7 +102,6 @@ struct SosArgs {
   unsigned spin_limit;         // look-back polls before the self-compute fallback
   unsigned agg_only;           // testing: tiles after a row's first publish no inclusive state
   uint64_t *status;            // [B, S, tiles, kStride] status words of this call
-  int vec_ok;
   int kept_step;               // gradient backward: sections whose input stays in LDS (0: none)
   int out_lds;                 // gradient backward: kept slot 0 holds the output's LDS transpose
 };
@@ -698,7 +697,7 @@ __device__ __noinline__ Vec2<typename Wide<E>::type> sos_prefix_fallback(const S
     const int64_t t0 = REV ? row_end - off - int64_t(lane + 1) * K : off + int64_t(lane) * K;
     const int64_t t0s[1] = {t0};
     E u[1][K];
-    load_chunk<E, K>(inrow, t0, T, a.vec_ok != 0, u[0], zero);
+    load_chunk<E, K>(inrow, t0, T, u[0], zero);
     for (int i = 0; i < n; ++i) {
       const int s = REV ? S - 1 - i : i;
       const SosSec<E> q = load_sec(a, b, s);
@@ -815,7 +814,6 @@ __global__ __launch_bounds__(Sh::kThreads, (kSosMinWaves<E, REV>)) void sos_kern
   const int64_t qf = REV ? tiles - 1 - qs : qs;  // position along time
   const int64_t T = a.T_len;
   const int S = a.S;
-  const bool vec = a.vec_ok != 0;
   // the row's state before its first step in scan order; backward it is
   // dL/dzf only when no padded step t = T carries it
   const bool row_virt = !REV || (T % Sh::kTile) == 0;
@@ -887,13 +885,13 @@ __global__ __launch_bounds__(Sh::kThreads, (kSosMinWaves<E, REV>)) void sos_kern
 
   E U[R][K];  // forward: input of the current section;  backward: its upstream gradient
 #pragma unroll
-  for (int r = 0; r < R; ++r) load_chunk<E, K>(a.in + b * T, chunk0(r), T, vec, U[r], zero);
+  for (int r = 0; r < R; ++r) load_chunk<E, K>(a.in + b * T, chunk0(r), T, U[r], zero);
   // forward values of the current section (x is read again from memory
   // where a re-derivation starts from it, not held in registers)
   E F[GRAD ? R : 1][GRAD ? K : 1];
   if constexpr (GRAD) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) load_chunk<E, K>(a.x + b * T, chunk0(r), T, vec, F[r], zero);
+    for (int r = 0; r < R; ++r) load_chunk<E, K>(a.x + b * T, chunk0(r), T, F[r], zero);
   }
   if constexpr (ONE) {  // x into the output's slot, for the visit
 #pragma unroll
@@ -973,7 +971,7 @@ __global__ __launch_bounds__(Sh::kThreads, (kSosMinWaves<E, REV>)) void sos_kern
           for (int k = 0; k < K; ++k) Uf[r][k] = src[((w * R + r) * K + k) * 64 + lane];
       } else {
 #pragma unroll
-        for (int r = 0; r < R; ++r) load_chunk<E, K>(a.x + b * T, chunk0(r), T, vec, Uf[r], zero);
+        for (int r = 0; r < R; ++r) load_chunk<E, K>(a.x + b * T, chunk0(r), T, Uf[r], zero);
       }
       for (int j = j0; j < s; ++j) {
         const SosSec<E> qj = load_sec(a, b, j);
@@ -1049,13 +1047,13 @@ __global__ __launch_bounds__(Sh::kThreads, (kSosMinWaves<E, REV>)) void sos_kern
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int64_t blk0 = chunk0(r) - int64_t(pl) * K;  // the round's block, lowest time first
-      if (kOutLds && wb != nullptr && vec && blk0 + 64 * K <= T) {
+      if (kOutLds && wb != nullptr && blk0 + 64 * K <= T) {
         if constexpr (kOutLds) {
           lds_put_chunk<E, K>(wb, pl, U[r]);
-          lds_flush<kNVo>(reinterpret_cast<uint4 *>(a.out + b * T + blk0), wb, lane, true);
+          lds_flush<kNVo>(a.out + b * T + blk0, wb, lane, true);
         }
       } else {
-        store_chunk<E, K>(a.out + b * T, chunk0(r), T, vec, U[r]);
+        store_chunk<E, K>(a.out + b * T, chunk0(r), T, U[r]);
       }
     }
   }

@@ -67,7 +67,6 @@ bool ss_args(int64_t B, int64_t T, const SsFilter &f, const void *zi, const void
   const unsigned sl = g_spin_limit.load(std::memory_order_relaxed);
   a.spin_limit = sl ? sl : kDefaultSpinLimit;
   a.agg_only = g_agg_only.load(std::memory_order_relaxed) ? 1u : 0u;
-  a.vec_ok = (size_t(T) * sizeof(E)) % 16 == 0 && aligned16(x) && aligned16(y);
   return true;
 }
 
@@ -136,8 +135,6 @@ int ss_fwd(int64_t B, int64_t T, const void *A, bool A_sh, const void *bv, bool 
   a.out_idx = out_idx;
   if (hs) {  // the states as well, in the same pass (the states-and-output mode)
     a.hs = static_cast<E *>(hs);
-    a.vec_hs = aligned16(hs) && (size_t(T) * sizeof(typename Alg::s_state)) % 16 == 0 && aligned16(x) &&
-               (size_t(T) * sizeof(E)) % 16 == 0;
     return rev ? ss_launch<Alg, true, kSsStatesY>(a, stream) : ss_launch<Alg, false, kSsStatesY>(a, stream);
   }
   return rev ? ss_launch<Alg, true>(a, stream) : ss_launch<Alg, false>(a, stream);
@@ -202,8 +199,6 @@ int ss_bwd(int64_t B, int64_t T, const SsModelArgs<typename Alg::elem> &mo, cons
     if (!ss_args<Alg>(B, T, f, zi, x, nullptr, nullptr, workspace, ws_bytes, p)) return PHS_ERR_WORKSPACE;
     set_model(p, false);
     p.hs = states;
-    p.vec_hs = aligned16(states) && (size_t(T) * sizeof(SS)) % 16 == 0 && aligned16(x) &&
-               (size_t(T) * sizeof(E)) % 16 == 0;
     int rc = PHS_OK;
     if (!hs_in) {
       rc = rev ? ss_launch<Alg, true, kSsStates>(p, stream) : ss_launch<Alg, false, kSsStates>(p, stream);
@@ -216,8 +211,6 @@ int ss_bwd(int64_t B, int64_t T, const SsModelArgs<typename Alg::elem> &mo, cons
     p.hs_fwd = states;
     p.x_fwd = static_cast<const E *>(x);
     p.gpart = gpart;
-    p.vec_hs = aligned16(states) && (size_t(T) * sizeof(SS)) % 16 == 0 && aligned16(x) &&
-               (size_t(T) * sizeof(E)) % 16 == 0;
     rc = rev ? ss_launch<Alg, false, kSsGrad>(p, stream) : ss_launch<Alg, true, kSsGrad>(p, stream);
     if (rc != PHS_OK) return rc;
   }
@@ -264,9 +257,6 @@ int ss_filtfilt(int64_t B, int64_t T, const SsFilter &f, int mode, int64_t e, co
   using E = typename Alg::elem;
   using SS = typename Alg::s_state;
   const bool keep = h1 && h2;
-  auto vec_states = [&](const void *hs, const void *xf) {
-    return aligned16(hs) && (size_t(T) * sizeof(SS)) % 16 == 0 && aligned16(xf) && (size_t(T) * sizeof(E)) % 16 == 0;
-  };
   if (ws_bytes < filtfilt_ws_bytes<E>(B, T)) return PHS_ERR_WORKSPACE;  // the documented size, any order
   char *m = static_cast<char *>(mid);
   E *y1 = reinterpret_cast<E *>(m);
@@ -279,7 +269,6 @@ int ss_filtfilt(int64_t B, int64_t T, const SsFilter &f, int mode, int64_t e, co
   p.pad_len = e;
   if (keep) {
     p.hs = static_cast<E *>(h1);
-    p.vec_hs = vec_states(h1, x);
   }
   int rc = keep ? ss_launch<Alg, false, kSsStatesY>(p, stream) : ss_launch<Alg, false>(p, stream);
   if (rc != PHS_OK) return rc;
@@ -291,7 +280,6 @@ int ss_filtfilt(int64_t B, int64_t T, const SsFilter &f, int mode, int64_t e, co
   p.pad_len = e;
   if (keep) {
     p.hs = static_cast<E *>(h2);
-    p.vec_hs = vec_states(h2, y1);
     return ss_launch<Alg, true, kSsStatesY>(p, stream);
   }
   return ss_launch<Alg, true>(p, stream);
@@ -399,9 +387,6 @@ int ss_filtfilt_bwd(int64_t B, int64_t T, const SsFilter &f, int mode, int64_t e
   E *y1 = nullptr, *zf1 = nullptr;
   SS *h1 = nullptr, *h2 = nullptr;
   C *gpart = nullptr, *rowsum1 = nullptr, *rowsum2 = nullptr;
-  auto vec_states = [&](const void *hs, const void *xf) {
-    return aligned16(hs) && (size_t(T) * sizeof(SS)) % 16 == 0 && aligned16(xf) && (size_t(T) * sizeof(E)) % 16 == 0;
-  };
   if (coef) {
     y1 = static_cast<E *>(at(L.y1));
     zf1 = static_cast<E *>(at(L.zf1));
@@ -436,7 +421,6 @@ int ss_filtfilt_bwd(int64_t B, int64_t T, const SsFilter &f, int mode, int64_t e
     p.pad_mode = mode;
     p.pad_len = e;
     p.hs = reinterpret_cast<E *>(h1);
-    p.vec_hs = vec_states(h1, x);
     if ((rc = ss_launch<Alg, false, kSsStatesY>(p, stream)) != PHS_OK) return rc;
     p = SsArgs<Alg>{};
     if (!ss_args<Alg>(B, T, f, nullptr, y1, nullptr, nullptr, workspace, ws_bytes, p)) return PHS_ERR_WORKSPACE;
@@ -446,7 +430,6 @@ int ss_filtfilt_bwd(int64_t B, int64_t T, const SsFilter &f, int mode, int64_t e
     p.pad_mode = mode;
     p.pad_len = e;
     p.hs = reinterpret_cast<E *>(h2);
-    p.vec_hs = vec_states(h2, y1);
     if ((rc = ss_launch<Alg, true, kSsStates>(p, stream)) != PHS_OK) return rc;
   }
   // pass 2's adjoint over the interior (ascending time)
@@ -458,7 +441,6 @@ int ss_filtfilt_bwd(int64_t B, int64_t T, const SsFilter &f, int mode, int64_t e
     p.hs_fwd = reinterpret_cast<const E *>(h2);
     p.x_fwd = y1;
     p.gpart = gpart;
-    p.vec_hs = vec_states(h2, y1);
     if ((rc = ss_launch<Alg, false, kSsGrad>(p, stream)) != PHS_OK) return rc;
     hipLaunchKernelGGL(ss_grad_rows_kernel<Alg>, dim3(unsigned(B)), dim3(kSsReduceThreads), 0, stream,
                        static_cast<const C *>(gpart), tiles * SsShape<Alg, kSsGrad>::kWaves, rowsum2);
@@ -478,7 +460,6 @@ int ss_filtfilt_bwd(int64_t B, int64_t T, const SsFilter &f, int mode, int64_t e
     p.hs_fwd = reinterpret_cast<const E *>(h1);
     p.x_fwd = static_cast<const E *>(x);
     p.gpart = gpart;
-    p.vec_hs = vec_states(h1, x);
     if ((rc = ss_launch<Alg, true, kSsGrad>(p, stream)) != PHS_OK) return rc;
     hipLaunchKernelGGL(ss_grad_rows_kernel<Alg>, dim3(unsigned(B)), dim3(kSsReduceThreads), 0, stream,
                        static_cast<const C *>(gpart), tiles * SsShape<Alg, kSsGrad>::kWaves, rowsum1);

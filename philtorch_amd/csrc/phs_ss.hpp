@@ -85,7 +85,6 @@ struct SsArgs {
   E *hs;
   const E *hs_fwd, *x_fwd;
   typename Wide<E>::type *gpart;
-  int vec_hs;         // 16-byte state chunks (T M sizeof(E) % 16 == 0, aligned)
   int64_t B, T_len, tiles_per_row;
   unsigned long long *claims;
   unsigned tiles, per_stripe, spin_limit;
@@ -93,7 +92,6 @@ struct SsArgs {
   uint64_t b_magic;   // tile id -> row by multiply and shift (row_split)
   unsigned b_shift;
   uint64_t *status;
-  int vec_ok;
   // plain forward of a second-order model (nullable): the state entering
   // every ckpt_every-th step, in compute precision, [B, n_ckpt] (the
   // checkpoints the fused cascade's gradient backward reads at one section)
@@ -153,16 +151,16 @@ struct SsShape {
 // T - s0, read (and written) in descending time.  Positions past the row
 // read 0 and are not written.  The bounds-checked paths assign in branches
 // (no select between a global and a private address).  kFull: the chunk
-// is known to be in range and aligned, only the vector form is compiled.
+// is known to be in range, only the vector form is compiled.
 template <bool REV, typename E, int K, bool kFull = false>
-__device__ __forceinline__ void ss_load(const E *row, int64_t s0, int64_t T, bool vec, E (&out)[K]) {
+__device__ __forceinline__ void ss_load(const E *row, int64_t s0, int64_t T, E (&out)[K]) {
   if constexpr (!REV) {
-    load_chunk<E, K, kFull>(row, s0, T, vec, out, E{});
+    load_chunk<E, K, kFull>(row, s0, T, out, E{});
   } else {
     const int64_t base = T - s0 - K;  // lowest time of the chunk
-    if (kFull || (vec && base >= 0)) {
+    if (kFull || base >= 0) {
       E tmp[K];
-      load_chunk<E, K>(row, base, T, true, tmp, E{});
+      load_chunk<E, K, true>(row, base, T, tmp, E{});
 #pragma unroll
       for (int k = 0; k < K; ++k) out[k] = tmp[K - 1 - k];
     } else {
@@ -179,17 +177,17 @@ __device__ __forceinline__ void ss_load(const E *row, int64_t s0, int64_t T, boo
 }
 
 template <bool REV, typename E, int K, bool kFull = false>
-__device__ __forceinline__ void ss_store(E *row, int64_t s0, int64_t T, bool vec, const E (&v)[K]) {
+__device__ __forceinline__ void ss_store(E *row, int64_t s0, int64_t T, const E (&v)[K]) {
   static_assert(K * sizeof(E) % 16 == 0, "whole 16-byte vectors");
   if constexpr (!REV) {
-    store_chunk<E, K, kFull>(row, s0, T, vec, v);
+    store_chunk<E, K, kFull>(row, s0, T, v);
   } else {
     const int64_t base = T - s0 - K;
-    if (kFull || (vec && base >= 0)) {
+    if (kFull || base >= 0) {
       E tmp[K];
 #pragma unroll
       for (int k = 0; k < K; ++k) tmp[k] = v[K - 1 - k];
-      store_chunk<E, K>(row, base, T, true, tmp);
+      store_chunk<E, K, true>(row, base, T, tmp);
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
@@ -605,7 +603,7 @@ __device__ __noinline__ typename Alg::state ss_prefix_fallback(const SsArgs<Alg>
   for (int64_t off = 0; off < span; off += 64 * K) {
     ss_reload_tables();
     E xs[K];
-    ss_load<REV, E, K>(xrow, off + int64_t(ss_scan_lane<REV>(lane)) * K, a.T_len, a.vec_ok != 0, xs);
+    ss_load<REV, E, K>(xrow, off + int64_t(ss_scan_lane<REV>(lane)) * K, a.T_len, xs);
     typename Alg::state v[1] = {ss_lane_fold<Alg, K>(m, xs)};
     ss_lane_scan<Alg, 1, REV>(v, lane, tab->pw);
     st = Alg::affine(tab->pw[6], st, read_lane(v[0], ss_last_lane<REV>()));
@@ -902,7 +900,6 @@ __global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>
   }
 
   // ================= data waves
-  const bool vec = a.vec_ok != 0;
   const E *xrow = a.x + b * T;
   const int64_t seg0 = q * Sh::kTile + int64_t(w) * Sh::kWaveSeg;
   const int sl = ss_scan_lane<REV>(lane);
@@ -913,8 +910,8 @@ __global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>
   // and fp64 (register spills at order 4) take the model from LDS.
   constexpr bool kOwnModel = V::M >= 3 && sizeof(E) == 4;
   // The data path, compiled twice: kFull for tiles wholly inside the row
-  // with aligned rows (vector loads and stores only, so each round's fold
-  // waits for its own loads), and the bounds-checked form.
+  // (vector loads and stores only, so each round's fold waits for its own
+  // loads), and the bounds-checked form.
   auto data_path = [&](auto full_c) {
     constexpr bool kFull = decltype(full_c)::value;
     issue_barrier();  // the look-back wave has issued the model's reads
@@ -925,7 +922,7 @@ __global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       t0s[r] = seg0 + int64_t(r) * 64 * K + int64_t(sl) * K;
-      ss_load<REV, E, K, kFull>(xrow, t0s[r], T, vec, X[r]);
+      ss_load<REV, E, K, kFull>(xrow, t0s[r], T, X[r]);
     }
     // ---- pass 1: every map's matrix part is a known power of A, so only the
     // vector parts are scanned.  Steps past the row's end take a zero input
@@ -990,7 +987,6 @@ __global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>
     // vectors
     constexpr int G = MODE == kSsPlain ? int(16 / sizeof(E)) : ss_state_group<Alg>();
     static_assert(K % G == 0 && G * sizeof(E) % 16 == 0, "groups of whole output vectors");
-    const bool vh = a.vec_hs != 0;
     SsGrad<Alg, E> lacc;
     if constexpr (MODE == kSsGrad) {
 #pragma unroll
@@ -1019,8 +1015,8 @@ __global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>
         E Xg[G];
         E Og[G];
         if constexpr (MODE == kSsGrad) {
-          ss_load<REV, SS, G>(reinterpret_cast<const SS *>(a.hs_fwd) + b * T, t0s[r] + g0, T, vh, Hg);
-          ss_load<REV, E, G>(a.x_fwd + b * T, t0s[r] + g0, T, vh, Xg);
+          ss_load<REV, SS, G>(reinterpret_cast<const SS *>(a.hs_fwd) + b * T, t0s[r] + g0, T, Hg);
+          ss_load<REV, E, G>(a.x_fwd + b * T, t0s[r] + g0, T, Xg);
         }
 #pragma unroll
         for (int k2 = 0; k2 < G; ++k2) {
@@ -1044,20 +1040,20 @@ __global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>
         if constexpr (kFull && kHLds)
           ss_lds_put<kNVh, REV, K>(s_ht + w * 64 * kNVh, lane, g0, Hg);
         else if constexpr (kStates)
-          ss_store<REV, SS, G>(reinterpret_cast<SS *>(a.hs) + b * T, t0s[r] + g0, T, vh, Hg);
+          ss_store<REV, SS, G>(reinterpret_cast<SS *>(a.hs) + b * T, t0s[r] + g0, T, Hg);
         if constexpr (kFull && kYLds)
           ss_lds_put<kNVy, REV, K>(s_yt + w * 64 * kNVy, lane, g0, Og);
         else if (want_y)
-          ss_store<REV, E, G, kFull>(a.y + b * T, t0s[r] + g0, T, vec, Og);
+          ss_store<REV, E, G, kFull>(a.y + b * T, t0s[r] + g0, T, Og);
       }
       // the round's block, lowest time first
       const int64_t p0 = seg0 + int64_t(r) * 64 * K;  // first scan position of the round
       const int64_t tb = REV ? T - p0 - 64 * K : p0;
       if constexpr (kFull && kHLds)
-        lds_flush<kNVh>(reinterpret_cast<uint4 *>(reinterpret_cast<SS *>(a.hs) + b * T + tb),
+        lds_flush<kNVh>(reinterpret_cast<SS *>(a.hs) + b * T + tb,
                            s_ht + w * 64 * kNVh, lane, true);
       if constexpr (kFull && kYLds)
-        lds_flush<kNVy>(reinterpret_cast<uint4 *>(a.y + b * T + tb), s_yt + w * 64 * kNVy, lane, want_y);
+        lds_flush<kNVy>(a.y + b * T + tb, s_yt + w * 64 * kNVy, lane, want_y);
     }
     if constexpr (MODE == kSsGrad) {
       // the wave's sums, in a fixed order, one partial per (row, tile, wave)
@@ -1078,8 +1074,7 @@ __global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>
       }
     }
   };
-  // the state modes' full path also needs 16-byte state rows (vec_hs)
-  if (vec && (!kStates || a.vec_hs) && (q + 1) * Sh::kTile <= T)
+  if ((q + 1) * Sh::kTile <= T)
     data_path(std::true_type{});
   else
     data_path(std::false_type{});
