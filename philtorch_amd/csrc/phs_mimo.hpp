@@ -334,25 +334,8 @@ __global__ __launch_bounds__(MimoShape<Alg>::kThreads, MimoShape<Alg>::kMinWaves
 
   if (w == kWaves) {
     // ================= look-back wave: power tables, then the look-back
-    {
-      const typename Alg::s_coef Arow = V::load_mat(a.A + b * a.A_stride);
-      typename Alg::coef P = ss_pow2<Alg>(Arow, __builtin_ctz(K));
-#pragma unroll
-      for (int i = 0; i < 6; ++i) {
-        if (lane == 0) s_tab.pw[i] = P;
-        P = Alg::cmul(P, P);
-      }
-      if (lane == 0) s_tab.pw[6] = P;  // A^(64 K), a wave's span
-      if (lane == 0) s_tab.pw[7] = P;
-      typename Alg::coef G = P;  // A^(kWaves 64 K), a tile
-#pragma unroll
-      for (int j = 1; j < kWaves; ++j) G = Alg::cmul(P, G);
-#pragma unroll
-      for (int j = 0; j < 7; ++j) {
-        if (lane == 0) s_tab.gp[j] = G;
-        G = Alg::cmul(G, G);
-      }
-    }
+    ss_build_powers<Alg, K, 1, kWaves>(reinterpret_cast<const typename Alg::s_coef *>(a.A + b * a.A_stride), &s_tab,
+                                       lane);
     __syncthreads();  // power tables
     tag = claim_tag(a.claims, a.per_stripe, lane);
     uint64_t *row_status = a.status + b * a.tiles_per_row * St::kStride;

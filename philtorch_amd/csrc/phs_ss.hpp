@@ -491,14 +491,6 @@ __device__ __forceinline__ typename Alg::state ss_filtfilt_entry(const SsArgs<Al
   return Alg::load_s(u.s);
 }
 
-// A^(2^n) in compute precision.
-template <class Alg>
-__device__ __forceinline__ typename Alg::coef ss_pow2(const typename Alg::s_coef &A, int n) {
-  typename Alg::coef P = Alg::load_c(A);
-  for (int i = 0; i < n; ++i) P = Alg::cmul(P, P);
-  return P;
-}
-
 // A lane's K steps from a zero state, sum_k A^(K-1-k) b x[k] (the vector
 // part of its map; the matrix part is A^K).
 template <class Alg, int K>
@@ -532,6 +524,71 @@ struct SsPowers {
   typename Alg::coef pw[8];
   typename Alg::coef gp[7];
 };
+
+// One 4 x 4 fp64 matrix (orders 3 and 4, order 3 padded with zeros) held one
+// element a lane, as n = P[i][j] and t = P[j][i] with i = lane / 16, j = lane
+// % 4 (the four blocks lane / 4 % 4 hold the same): the operand layouts of
+// v_mfma_f64_4x4x4, which reads its left matrix as t and its right one as n
+// and returns n.  A product is two such instructions (its n and its t) where
+// every lane doing the whole product itself takes M^3 FMAs, 64 at order 4;
+// the power tables are a chain of some twenty of them that every tile waits
+// for.  Order 4, before -> after (us): lfilter of 16 x 480000 fp32 46.6 ->
+// 41.0, trained 180.6 -> 152.6, of 16 x 240000 fp64 46.3 -> 36.4, zero-phase
+// 98.0 -> 84.2, the multi-input model of 16 x 480000 (2 in, 2 out) 112.1 ->
+// 103.4.  Needs the whole wave active.
+struct Pow4 {
+  double n, t;
+};
+__device__ __forceinline__ Pow4 pow4_mul(const Pow4 &p, const Pow4 &q) {
+  return {__builtin_amdgcn_mfma_f64_4x4x4f64(p.t, q.n, 0.0, 0, 0, 0),
+          __builtin_amdgcn_mfma_f64_4x4x4f64(q.n, p.t, 0.0, 0, 0, 0)};
+}
+
+// The power tables of one row's A by one wave: pw from A^K on (K, R powers
+// of two), gp for a tile of W wave segments.
+template <class Alg, int K, int R, int W>
+__device__ __forceinline__ void ss_build_powers(const typename Alg::s_coef *A, SsPowers<Alg> *tab, int lane) {
+  constexpr int M = SsView<Alg>::M;
+  static_assert((K & (K - 1)) == 0 && (R & (R - 1)) == 0, "powers by squaring");
+  // build(P, mul, put): the chain itself, for either form of a matrix
+  auto build = [&](auto P, auto &&mul, auto &&put) {
+#pragma unroll
+    for (int k = 1; k < K; k <<= 1) P = mul(P, P);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      put(tab->pw[i], P);
+      P = mul(P, P);
+    }
+    put(tab->pw[6], P);
+#pragma unroll
+    for (int r = 1; r < R; r <<= 1) P = mul(P, P);
+    put(tab->pw[7], P);
+    auto G = P;
+#pragma unroll
+    for (int j = 1; j < W; ++j) G = mul(P, G);
+#pragma unroll
+    for (int j = 0; j < 7; ++j) {
+      put(tab->gp[j], G);
+      if (j < 6) G = mul(G, G);
+    }
+  };
+  if constexpr (M >= 3) {
+    const int i = lane >> 4, j = lane & 3;
+    const bool in = i < M && j < M;
+    const typename Alg::elem *e = reinterpret_cast<const typename Alg::elem *>(A);
+    Pow4 P{0.0, 0.0};
+    if (in) P = {double(e[i * M + j]), double(e[j * M + i])};
+    const bool mine = in && (lane & 12) == 0;
+    build(P, pow4_mul, [&](typename Alg::coef &dst, const Pow4 &p) {
+      if (mine) reinterpret_cast<double *>(&dst)[i * M + j] = p.n;
+    });
+  } else {
+    build(Alg::load_c(*A), [](const auto &p, const auto &q) { return Alg::cmul(p, q); },
+          [&](typename Alg::coef &dst, const typename Alg::coef &p) {
+            if (lane == 0) dst = p;
+          });
+  }
+}
 
 // The power tables live in LDS and are read where they are used: a compiler
 // barrier at the top of each loop keeps their loads from being hoisted out
@@ -843,27 +900,8 @@ __global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>
       const SsModel<Alg> mrow = ss_model<Alg, MODE == kSsGrad>(a, b);
       issue_barrier();
       if (lane == 0) s_model = mrow;
-      typename Alg::coef P = ss_pow2<Alg>(mrow.A, __builtin_ctz(K));
-#pragma unroll
-      for (int i = 0; i < 6; ++i) {
-        if (lane == 0) s_tab.pw[i] = P;
-        P = Alg::cmul(P, P);
-      }
-      if (lane == 0) s_tab.pw[6] = P;
-#pragma unroll
-      for (int r = 1; r < R; r <<= 1) P = Alg::cmul(P, P);
-      if (lane == 0) s_tab.pw[7] = P;
-      {  // G = A^(kWaves * 64 K R)
-        typename Alg::coef G = P;
-#pragma unroll
-        for (int j = 1; j < kWaves; ++j) G = Alg::cmul(P, G);
-        P = G;
-      }
-#pragma unroll
-      for (int j = 0; j < 7; ++j) {
-        if (lane == 0) s_tab.gp[j] = P;
-        P = Alg::cmul(P, P);
-      }
+      wave_sync();
+      ss_build_powers<Alg, K, R, kWaves>(&s_model.A, &s_tab, lane);
     }
     __syncthreads();  // power tables
     tag = claim_tag(a.claims, a.per_stripe, lane);
