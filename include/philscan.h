@@ -651,6 +651,16 @@ int phs_mimo_ss_rev(int dtype, int M, int F, int P, int64_t B, int64_t T, const 
                     const void *Cm, const void *Dm, int shared, const void *zi, const void *x, void *y, void *zf,
                     void *workspace, size_t workspace_bytes, void *stream);
 
+/* phs_mimo_ss_fwd (reverse != 0: phs_mimo_ss_rev) that also writes hs
+ * [B,T,M], the state before every step, in the same pass (no counterpart in
+ * the reference, whose autograd saves the composed route's tensors): the
+ * states the coefficient gradients read (phs_mimo_ss_grad_sums), so a
+ * caller need not run the model again with C the identity.  y and zf equal
+ * those calls' bit for bit. */
+int phs_mimo_ss_hs(int dtype, int M, int F, int P, int64_t B, int64_t T, const void *A, const void *Bm,
+                   const void *Cm, const void *Dm, int shared, const void *zi, const void *x, void *y, void *zf,
+                   void *hs, int reverse, void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---- Multi-input, multi-output LPV (time-varying A) state space of order
  * M = 1..4 with F = 1..4 inputs and P = 1..4 outputs per step, fused.
  * Replaces philtorch.lpv.state_space (philtorch/lpv/ssm.py:337-581) for a

@@ -11,7 +11,9 @@ namespace {
 
 template <class Alg>
 size_t mimo_ws_bytes(int64_t B, int64_t T) {
-  const int64_t tiles = (T + MimoShape<Alg>::kTile - 1) / MimoShape<Alg>::kTile;
+  // the shortest tile of any input width
+  constexpr int64_t tile = std::min<int64_t>(MimoShape<Alg, 1>::kTile, MimoShape<Alg, kMimoMaxIO>::kTile);
+  const int64_t tiles = (T + tile - 1) / tile;
   return align_up(align_up(kHeaderBytes) + size_t(B) * size_t(tiles) * SsStatus<Alg>::kStride * sizeof(uint64_t));
 }
 
@@ -25,14 +27,14 @@ __global__ __launch_bounds__(256) void mimo_empty_zf_kernel(const E *zi, int64_t
   if (i < n) zf[i] = zi ? zi[i] : E(0);
 }
 
-template <class Alg>
-int mimo_ss(int F, int P, int64_t B, int64_t T, const void *A, const void *Bm, const void *Cm, const void *Dm,
-            int shared, const void *zi, const void *x, void *y, void *zf, void *workspace, size_t ws_bytes, bool rev,
-            hipStream_t stream) {
+template <class Alg, int F>
+int mimo_ss_f(int P, int64_t B, int64_t T, const void *A, const void *Bm, const void *Cm, const void *Dm, int shared,
+              const void *zi, const void *x, void *y, void *zf, void *workspace, size_t ws_bytes, bool rev,
+              hipStream_t stream, void *hs) {
   using E = typename Alg::elem;
-  using Sh = MimoShape<Alg>;
+  using Sh = MimoShape<Alg, F>;
   constexpr int M = SsView<Alg>::M;
-  if (B < 0 || T < 0 || F < 1 || F > kMimoMaxIO || P < 1 || P > kMimoMaxIO) return PHS_ERR_INVALID;
+  if (B < 0 || T < 0 || P < 1 || P > kMimoMaxIO) return PHS_ERR_INVALID;
   if (shared & ~(PHS_MIMO_A_SHARED | PHS_MIMO_B_SHARED | PHS_MIMO_C_SHARED | PHS_MIMO_D_SHARED))
     return PHS_ERR_INVALID;
   if (B == 0) return PHS_OK;
@@ -61,8 +63,8 @@ int mimo_ss(int F, int P, int64_t B, int64_t T, const void *A, const void *Bm, c
   a.d_stride = (shared & PHS_MIMO_D_SHARED) ? 0 : int64_t(P) * F;
   a.F = F;
   a.P = P;
-  a.f_magic = io_magic(F);
-  a.p_magic = io_magic(P);
+  a.p_magic18 = unsigned(((1u << 18) + unsigned(P) - 1u) / unsigned(P));
+  a.hs = static_cast<E *>(hs);
   a.zi = static_cast<const E *>(zi);
   a.x = static_cast<const E *>(x);
   a.y = static_cast<E *>(y);
@@ -79,11 +81,35 @@ int mimo_ss(int F, int P, int64_t B, int64_t T, const void *A, const void *Bm, c
   a.spin_limit = sl ? sl : kDefaultSpinLimit;
   a.agg_only = g_agg_only.load(std::memory_order_relaxed) ? 1u : 0u;
   const dim3 grid(a.per_stripe * kStripes), block(Sh::kThreads);
-  if (rev)
-    launch_kernel((mimo_ss_kernel<Alg, true>), grid, block, 0, stream, a);
-  else
-    launch_kernel((mimo_ss_kernel<Alg, false>), grid, block, 0, stream, a);
+  const unsigned lds = unsigned(Sh::lds_bytes(P, hs != nullptr));
+  if (hs) {
+    if (rev)
+      launch_kernel((mimo_ss_kernel<Alg, F, true, true>), grid, block, lds, stream, a);
+    else
+      launch_kernel((mimo_ss_kernel<Alg, F, false, true>), grid, block, lds, stream, a);
+  } else if (rev) {
+    launch_kernel((mimo_ss_kernel<Alg, F, true, false>), grid, block, lds, stream, a);
+  } else {
+    launch_kernel((mimo_ss_kernel<Alg, F, false, false>), grid, block, lds, stream, a);
+  }
   return hipGetLastError() == hipSuccess ? PHS_OK : PHS_ERR_LAUNCH;
+}
+
+template <class Alg>
+int mimo_ss(int F, int P, int64_t B, int64_t T, const void *A, const void *Bm, const void *Cm, const void *Dm,
+            int shared, const void *zi, const void *x, void *y, void *zf, void *workspace, size_t ws_bytes, bool rev,
+            hipStream_t stream, void *hs = nullptr) {
+  auto run = [&](auto f) {
+    return mimo_ss_f<Alg, decltype(f)::value>(P, B, T, A, Bm, Cm, Dm, shared, zi, x, y, zf, workspace, ws_bytes, rev,
+                                              stream, hs);
+  };
+  switch (F) {
+    case 1: return run(std::integral_constant<int, 1>{});
+    case 2: return run(std::integral_constant<int, 2>{});
+    case 3: return run(std::integral_constant<int, 3>{});
+    case 4: return run(std::integral_constant<int, 4>{});
+    default: return PHS_ERR_INVALID;
+  }
 }
 
 // ---- the coefficient gradients, summed over time in one pass over the
@@ -573,11 +599,11 @@ int mimo_dispatch(int dtype, int M, Fn &&f) {
 
 int mimo_call(int dtype, int M, int F, int P, int64_t B, int64_t T, const void *A, const void *Bm, const void *Cm,
               const void *Dm, int shared, const void *zi, const void *x, void *y, void *zf, void *workspace,
-              size_t workspace_bytes, bool rev, void *stream) {
+              size_t workspace_bytes, bool rev, void *stream, void *hs = nullptr) {
   const hipStream_t st = static_cast<hipStream_t>(stream);
   return mimo_dispatch(dtype, M, [&](auto alg) {
     return mimo_ss<decltype(alg)>(F, P, B, T, A, Bm, Cm, Dm, shared, zi, x, y, zf, workspace, workspace_bytes, rev,
-                                  st);
+                                  st, hs);
   });
 }
 
@@ -608,6 +634,13 @@ int phs_mimo_ss_rev(int dtype, int M, int F, int P, int64_t B, int64_t T, const 
                     void *workspace, size_t workspace_bytes, void *stream) {
   return phs::mimo_call(dtype, M, F, P, B, T, A, Bm, Cm, Dm, shared, zi, x, y, zf, workspace, workspace_bytes, true,
                         stream);
+}
+
+int phs_mimo_ss_hs(int dtype, int M, int F, int P, int64_t B, int64_t T, const void *A, const void *Bm,
+                   const void *Cm, const void *Dm, int shared, const void *zi, const void *x, void *y, void *zf,
+                   void *hs, int reverse, void *workspace, size_t workspace_bytes, void *stream) {
+  return phs::mimo_call(dtype, M, F, P, B, T, A, Bm, Cm, Dm, shared, zi, x, y, zf, workspace, workspace_bytes,
+                        reverse != 0, stream, hs);
 }
 
 size_t phs_lpv_mimo_ss_workspace_size(int dtype, int M, int64_t B, int64_t T) {

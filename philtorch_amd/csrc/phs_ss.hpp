@@ -545,15 +545,19 @@ __device__ __forceinline__ Pow4 pow4_mul(const Pow4 &p, const Pow4 &q) {
 }
 
 // The power tables of one row's A by one wave: pw from A^K on (K, R powers
-// of two), gp for a tile of W wave segments.
+// of two), gp for a tile of W wave segments; half (nullable): A^(K/2).
 template <class Alg, int K, int R, int W>
-__device__ __forceinline__ void ss_build_powers(const typename Alg::s_coef *A, SsPowers<Alg> *tab, int lane) {
+__device__ __forceinline__ void ss_build_powers(const typename Alg::s_coef *A, SsPowers<Alg> *tab, int lane,
+                                                typename Alg::coef *half = nullptr) {
   constexpr int M = SsView<Alg>::M;
   static_assert((K & (K - 1)) == 0 && (R & (R - 1)) == 0, "powers by squaring");
   // build(P, mul, put): the chain itself, for either form of a matrix
   auto build = [&](auto P, auto &&mul, auto &&put) {
 #pragma unroll
-    for (int k = 1; k < K; k <<= 1) P = mul(P, P);
+    for (int k = 1; k < K; k <<= 1) {
+      if (half && 2 * k == K) put(*half, P);
+      P = mul(P, P);
+    }
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
       put(tab->pw[i], P);
