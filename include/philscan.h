@@ -656,7 +656,8 @@ int phs_mimo_ss_rev(int dtype, int M, int F, int P, int64_t B, int64_t T, const 
  * the reference, whose autograd saves the composed route's tensors): the
  * states the coefficient gradients read (phs_mimo_ss_grad_sums), so a
  * caller need not run the model again with C the identity.  y and zf equal
- * those calls' bit for bit. */
+ * those calls'.  hs NULL: phs_mimo_ss_fwd / phs_mimo_ss_rev; with hs, P may
+ * be 0 (the states alone: Cm, Dm and y are not read). */
 int phs_mimo_ss_hs(int dtype, int M, int F, int P, int64_t B, int64_t T, const void *A, const void *Bm,
                    const void *Cm, const void *Dm, int shared, const void *zi, const void *x, void *y, void *zf,
                    void *hs, int reverse, void *workspace, size_t workspace_bytes, void *stream);

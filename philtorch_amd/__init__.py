@@ -926,7 +926,11 @@ if EXTENSION_LOADED and _has_op("mimo_ss"):
 
     def _mimo_ss_setup(ctx, inputs, output):
         ctx.reverse = bool(inputs[6]) if len(inputs) > 6 else False
-        ctx.save_for_backward(*inputs[:6])
+        # mimo_ss_states: the forward's states too, for the coefficient backward
+        hs = output[2] if len(output) > 2 else None
+        if hs is not None:
+            ctx.mark_non_differentiable(hs)
+        ctx.save_for_backward(*inputs[:6], hs)
         ctx.set_materialize_grads(False)
 
     if _has_op("mimo_ss_grad_sums"):
@@ -953,9 +957,9 @@ if EXTENSION_LOADED and _has_op("mimo_ss"):
         The coefficient gradients
             dL/dA = sum_t lambda[t+1] h[t]^T,  dL/dB = sum_t lambda[t+1] x[t]^T,
             dL/dC = sum_t g[t] h[t]^T,         dL/dD = sum_t g[t] x[t]^T
-        take the states h[t] (the forward again with C = I and no D) and the
-        adjoint states lambda[t+1] (the adjoint pass with output matrix I),
-        each one more mimo_ss pass, and philtorch::mimo_ss_grad_sums: the
+        take the states h[t] (kept by mimo_ss_states, else the forward again
+        for its states alone) and the adjoint states lambda[t+1] (the adjoint
+        pass for its states alone), and philtorch::mimo_ss_grad_sums: the
         four sums over time (and the rows, for a shared operand) in one pass
         over lambda, h, x and g.  Under create_graph: the gradient
         of the composite the fused kernel replaces (B x, the native scan,
@@ -963,7 +967,8 @@ if EXTENSION_LOADED and _has_op("mimo_ss"):
         recomputed from the inputs and differentiable again."""
         from .lti.ssm import _mimo_composite
 
-        inputs = ctx.saved_tensors
+        saved = ctx.saved_tensors
+        inputs, kept_hs = saved[:6], saved[6]
         A, B, C, D, zi, x = inputs
         needs = ctx.needs_input_grad
         out = [None] * 7
@@ -980,10 +985,9 @@ if EXTENSION_LOADED and _has_op("mimo_ss"):
             for i, g in zip(wrt, res):
                 out[i] = g if g is not None else torch.zeros_like(inputs[i])
             return tuple(out)
-        M = A.size(-1)
         g = gy if gy is not None else x.new_zeros(x.size(0), x.size(1), C.size(-2))
         At, Ct = A.mT.contiguous(), C.mT.contiguous()
-        eye = torch.eye(M, dtype=x.dtype, device=x.device)
+        states = torch.ops.philtorch.mimo_ss_states
         # lambda is wanted for A or B: its pass also gives grad_zi, and the
         # sums pass writes grad_x = B^T lambda + D^T g beside the sums
         lam_pass = needs[0] or needs[1]
@@ -996,9 +1000,9 @@ if EXTENSION_LOADED and _has_op("mimo_ss"):
                 out[4] = gzi if needs[4] and zi is not None else None
             hs = lam = None
             if needs[0] or needs[2]:
-                hs, _ = torch.ops.philtorch.mimo_ss(A, B, eye, None, zi, x, ctx.reverse)
+                hs = kept_hs if kept_hs is not None else states(A, B, C[..., :0, :], None, zi, x, ctx.reverse)[2]
             if lam_pass:
-                lam, gzi = torch.ops.philtorch.mimo_ss(At, Ct, eye, None, gzf, g, not ctx.reverse)
+                _, gzi, lam = states(At, Ct, At[..., :0, :], None, gzf, g, not ctx.reverse)
                 out[4] = gzi if needs[4] and zi is not None else None
         want = sum(1 << i for i in range(4) if needs[i] and inputs[i] is not None)
         if lam_pass and needs[5]:
@@ -1015,6 +1019,22 @@ if EXTENSION_LOADED and _has_op("mimo_ss"):
         return tuple(out)
 
     torch.library.register_autograd("philtorch::mimo_ss", _mimo_ss_backward, setup_context=_mimo_ss_setup)
+
+    if _has_op("mimo_ss_states"):
+
+        @torch.library.register_fake("philtorch::mimo_ss_states")
+        def _(A, B, C, D, zi, x, reverse=False):
+            M = A.shape[-1]
+            return (x.new_empty((x.shape[0], x.shape[1], C.shape[-2])), x.new_empty((x.shape[0], M)),
+                    x.new_empty((x.shape[0], x.shape[1], M)))
+
+        def _mimo_ss_states_backward(ctx, gy, gzf, ghs):
+            """mimo_ss's backward with the states the forward kept (hs is not
+            differentiable): no states pass."""
+            return _mimo_ss_backward(ctx, gy, gzf)
+
+        torch.library.register_autograd("philtorch::mimo_ss_states", _mimo_ss_states_backward,
+                                        setup_context=_mimo_ss_setup)
 
 if EXTENSION_LOADED and _has_op("lpv_mimo_ss"):
     # LPV state space (A[t]) with F inputs and P outputs per step (F, P <= 4),

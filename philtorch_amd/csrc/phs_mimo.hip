@@ -34,7 +34,7 @@ int mimo_ss_f(int P, int64_t B, int64_t T, const void *A, const void *Bm, const 
   using E = typename Alg::elem;
   using Sh = MimoShape<Alg, F>;
   constexpr int M = SsView<Alg>::M;
-  if (B < 0 || T < 0 || P < 1 || P > kMimoMaxIO) return PHS_ERR_INVALID;
+  if (B < 0 || T < 0 || P < (hs ? 0 : 1) || P > kMimoMaxIO) return PHS_ERR_INVALID;
   if (shared & ~(PHS_MIMO_A_SHARED | PHS_MIMO_B_SHARED | PHS_MIMO_C_SHARED | PHS_MIMO_D_SHARED))
     return PHS_ERR_INVALID;
   if (B == 0) return PHS_OK;
@@ -47,7 +47,7 @@ int mimo_ss_f(int P, int64_t B, int64_t T, const void *A, const void *Bm, const 
     }
     return PHS_OK;
   }
-  if (!A || !Bm || !Cm || !x || !y) return PHS_ERR_INVALID;
+  if (!A || !Bm || !x || (P > 0 && (!Cm || !y))) return PHS_ERR_INVALID;
   const int64_t tiles_per_row = (T + Sh::kTile - 1) / Sh::kTile;
   if (double(B) * double(tiles_per_row) >= 2147483648.0) return PHS_ERR_INVALID;
   if (!workspace || ws_bytes < mimo_ws_bytes<Alg>(B, T)) return PHS_ERR_WORKSPACE;
@@ -57,13 +57,13 @@ int mimo_ss_f(int P, int64_t B, int64_t T, const void *A, const void *Bm, const 
   a.A_stride = (shared & PHS_MIMO_A_SHARED) ? 0 : M * M;
   a.Bm = static_cast<const E *>(Bm);
   a.b_stride = (shared & PHS_MIMO_B_SHARED) ? 0 : int64_t(M) * F;
-  a.Cm = static_cast<const E *>(Cm);
-  a.c_stride = (shared & PHS_MIMO_C_SHARED) ? 0 : int64_t(P) * M;
-  a.Dm = static_cast<const E *>(Dm);
+  a.Cm = static_cast<const E *>(P > 0 ? Cm : A);  // without outputs an in-bounds stand-in, not used
+  a.c_stride = P == 0 ? a.A_stride : (shared & PHS_MIMO_C_SHARED) ? 0 : int64_t(P) * M;
+  a.Dm = P > 0 ? static_cast<const E *>(Dm) : nullptr;
   a.d_stride = (shared & PHS_MIMO_D_SHARED) ? 0 : int64_t(P) * F;
   a.F = F;
   a.P = P;
-  a.p_magic18 = unsigned(((1u << 18) + unsigned(P) - 1u) / unsigned(P));
+  a.p_magic18 = P > 0 ? unsigned(((1u << 18) + unsigned(P) - 1u) / unsigned(P)) : 0u;
   a.hs = static_cast<E *>(hs);
   a.zi = static_cast<const E *>(zi);
   a.x = static_cast<const E *>(x);
@@ -156,7 +156,20 @@ struct SumStep {
 // and each thread keeps U steps' loads in flight per iteration.  (Staging
 // a block's steps through LDS with two barriers per 256 steps measured
 // slower still: 1111 us.)
-template <typename E, int WM, int WI, bool ALL>
+//
+// READ: how the operands are read.  kSumSome: those the wanted products
+// need; kSumAll: every one, unconditionally; kSumExact: every one, with F = P
+// = WI, each operand's step in whole vectors (a state row of order 4 is one
+// 16-byte load, not four).
+constexpr int kSumSome = 0, kSumAll = 1, kSumExact = 2;
+
+// N consecutive elements at element alignment
+template <typename E, int N>
+struct __attribute__((packed, aligned(4))) SumRow {
+  E e[N];
+};
+
+template <typename E, int WM, int WI, int READ>
 __global__ __launch_bounds__(kSumThreads) void mimo_grad_partial_kernel(GradSumIn<E> in, int64_t T, unsigned nblk,
                                                                         typename Wide<E>::type *part) {
   using C = typename Wide<E>::type;
@@ -175,7 +188,22 @@ __global__ __launch_bounds__(kSumThreads) void mimo_grad_partial_kernel(GradSumI
   const E *__restrict__ xrow = need_x ? in.x + b * T * F : nullptr;
   const E *__restrict__ grow = need_g ? in.g + b * T * P : nullptr;
   auto load = [&](int64_t t, SumStep<C, WM, WI> &s) {
-    if constexpr (ALL) {
+    if constexpr (READ == kSumExact) {
+      const SumRow<E, WM> l = reinterpret_cast<const SumRow<E, WM> *>(lrow)[t];
+      const SumRow<E, WM> h = reinterpret_cast<const SumRow<E, WM> *>(hrow)[t];
+      const SumRow<E, WI> u = reinterpret_cast<const SumRow<E, WI> *>(xrow)[t];
+      const SumRow<E, WI> g = reinterpret_cast<const SumRow<E, WI> *>(grow)[t];
+#pragma unroll
+      for (int i = 0; i < WM; ++i) {
+        s.l[i] = C(l.e[i]);
+        s.h[i] = C(h.e[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < WI; ++i) {
+        s.u[i] = C(u.e[i]);
+        s.g[i] = C(g.e[i]);
+      }
+    } else if constexpr (READ == kSumAll) {
       // every operand there: unconditional loads (an index past the width
       // reads its last element, zeroed after), so a thread's U steps of
       // loads are all in flight before the first use
@@ -485,8 +513,14 @@ int grad_sums(int M, int F, int P, int64_t B, int64_t T, const void *lam, const 
     const bool all = need_l && need_h && need_x && need_g;
     auto pick = [&](auto wm) {
       constexpr int WMc = decltype(wm)::value;
-      if (WI == 2) return all ? mimo_grad_partial_kernel<E, WMc, 2, true> : mimo_grad_partial_kernel<E, WMc, 2, false>;
-      return all ? mimo_grad_partial_kernel<E, WMc, 4, true> : mimo_grad_partial_kernel<E, WMc, 4, false>;
+      const bool exact = all && F == WI && P == WI;
+      if (WI == 2)
+        return exact ? mimo_grad_partial_kernel<E, WMc, 2, kSumExact>
+               : all ? mimo_grad_partial_kernel<E, WMc, 2, kSumAll>
+                     : mimo_grad_partial_kernel<E, WMc, 2, kSumSome>;
+      return exact ? mimo_grad_partial_kernel<E, WMc, 4, kSumExact>
+             : all ? mimo_grad_partial_kernel<E, WMc, 4, kSumAll>
+                   : mimo_grad_partial_kernel<E, WMc, 4, kSumSome>;
     };
     auto kern = M == 1   ? pick(std::integral_constant<int, 1>{})
                 : M == 2 ? pick(std::integral_constant<int, 2>{})

@@ -429,7 +429,9 @@ __device__ __noinline__ typename Alg::state mimo_prefix_fallback(const MimoArgs<
   return st;
 }
 
-// HS: also the state before every step into a.hs.
+// HS: also the state before every step into a.hs (with P = 0 the states
+// alone): 16 x 480000 fp32, order 4, 2 in 2 out, 76 us with the outputs and 62
+// without, where a second pass with C the identity took 95.
 template <class Alg, int F, bool REV, bool HS>
 __global__ __launch_bounds__((MimoShape<Alg, F>::kThreads), (MimoShape<Alg, F>::kMinWaves)) void mimo_ss_kernel(
     MimoArgs<Alg> a) {

@@ -1374,9 +1374,9 @@ std::vector<Tensor> mimo_ss_grad_sums_hip(const std::optional<Tensor> &lam, cons
 // (batch, P, M); D None, (P, F) or (batch, P, F); zi None or (batch, M);
 // y (batch, T, P).  reverse runs the model backwards in time
 // (phs_mimo_ss_rev), the form of its adjoint.
-std::tuple<Tensor, Tensor> mimo_ss_hip(const Tensor &A, const Tensor &Bm, const Tensor &Cm,
-                                       const std::optional<Tensor> &Dm, const std::optional<Tensor> &zi,
-                                       const Tensor &x, bool reverse) {
+std::tuple<Tensor, Tensor, Tensor> mimo_ss_impl(const Tensor &A, const Tensor &Bm, const Tensor &Cm,
+                                                const std::optional<Tensor> &Dm, const std::optional<Tensor> &zi,
+                                                const Tensor &x, bool reverse, bool keep_states) {
   TORCH_CHECK(x.dim() == 3, "philtorch::mimo_ss: x must be a 3D tensor (batch, time, features)");
   const int64_t B = x.size(0), T = x.size(1), F = x.size(2);
   TORCH_CHECK((A.dim() == 2 || A.dim() == 3) && A.size(-1) == A.size(-2),
@@ -1386,7 +1386,7 @@ std::tuple<Tensor, Tensor> mimo_ss_hip(const Tensor &A, const Tensor &Bm, const 
   TORCH_CHECK(F >= 1 && F <= 4, "philtorch::mimo_ss: 1 to 4 input features, got ", F);
   TORCH_CHECK(Cm.dim() == 2 || Cm.dim() == 3, "philtorch::mimo_ss: C must be (P, M) or (batch, P, M)");
   const int64_t P = Cm.size(-2);
-  TORCH_CHECK(P >= 1 && P <= 4, "philtorch::mimo_ss: 1 to 4 outputs, got ", P);
+  TORCH_CHECK(P >= (keep_states ? 0 : 1) && P <= 4, "philtorch::mimo_ss: 1 to 4 outputs, got ", P);
   TORCH_CHECK(x.scalar_type() == at::kFloat || x.scalar_type() == at::kDouble,
               "philtorch::mimo_ss: float32 or float64 only, got ", x.scalar_type());
   TORCH_CHECK(x.is_cuda(), "philtorch::mimo_ss: philtorch_amd runs on HIP devices only (got ", x.device(), ")");
@@ -1412,21 +1412,40 @@ std::tuple<Tensor, Tensor> mimo_ss_hip(const Tensor &A, const Tensor &Bm, const 
   Tensor dc = Dm ? Dm->contiguous() : Tensor(), zc = zi ? zi->contiguous() : Tensor();
   Tensor y = at::empty({B, T, P}, x.options());
   Tensor zf = at::empty({B, M}, x.options());
-  if (B == 0) return {y, zf};
+  Tensor hs = at::empty({keep_states ? B : 0, keep_states ? T : 0, M}, x.options());
+  if (B == 0) return {y, zf, hs};
   if (T == 0) {
     if (zi) zf.copy_(zc); else zf.zero_();
-    return {y, zf};
+    return {y, zf, hs};
   }
   const int shared = (A.dim() == 2 ? PHS_MIMO_A_SHARED : 0) | (Bm.dim() == 2 ? PHS_MIMO_B_SHARED : 0) |
                      (Cm.dim() == 2 ? PHS_MIMO_C_SHARED : 0) | (Dm && Dm->dim() == 2 ? PHS_MIMO_D_SHARED : 0);
   void *stream = stream_of(x);
   const Workspace ws = workspace_for(x, phs_mimo_ss_workspace_size(dt, int(M), B, T), stream);
-  check_status((reverse ? phs_mimo_ss_rev : phs_mimo_ss_fwd)(
-                   dt, int(M), int(F), int(P), B, T, Ac.const_data_ptr(), bc.const_data_ptr(), cc.const_data_ptr(),
-                   Dm ? dc.const_data_ptr() : nullptr, shared, zi ? zc.const_data_ptr() : nullptr,
-                   xc.const_data_ptr(), y.mutable_data_ptr(), zf.mutable_data_ptr(), ws.ptr, ws.bytes, stream),
+  check_status(phs_mimo_ss_hs(dt, int(M), int(F), int(P), B, T, Ac.const_data_ptr(), bc.const_data_ptr(),
+                              cc.const_data_ptr(), Dm ? dc.const_data_ptr() : nullptr, shared,
+                              zi ? zc.const_data_ptr() : nullptr, xc.const_data_ptr(), y.mutable_data_ptr(),
+                              zf.mutable_data_ptr(), keep_states ? hs.mutable_data_ptr() : nullptr, reverse ? 1 : 0,
+                              ws.ptr, ws.bytes, stream),
                "mimo_ss");
+  return {y, zf, hs};
+}
+
+std::tuple<Tensor, Tensor> mimo_ss_hip(const Tensor &A, const Tensor &Bm, const Tensor &Cm,
+                                       const std::optional<Tensor> &Dm, const std::optional<Tensor> &zi,
+                                       const Tensor &x, bool reverse) {
+  auto [y, zf, hs] = mimo_ss_impl(A, Bm, Cm, Dm, zi, x, reverse, false);
   return {y, zf};
+}
+
+// mimo_ss that also returns hs (batch, T, M), the state before every step
+// (the states the coefficient gradients read), from the same pass.  A C of no
+// rows (P = 0) asks for the states alone.
+std::tuple<Tensor, Tensor, Tensor> mimo_ss_states_hip(const Tensor &A, const Tensor &Bm, const Tensor &Cm,
+                                                      const std::optional<Tensor> &Dm,
+                                                      const std::optional<Tensor> &zi, const Tensor &x,
+                                                      bool reverse) {
+  return mimo_ss_impl(A, Bm, Cm, Dm, zi, x, reverse, true);
 }
 
 // ------------------------------------------------------------ CPU key
@@ -1631,6 +1650,8 @@ TORCH_LIBRARY(philtorch, m) {
         {at::Tag::pt2_compliant_tag});
   m.def("mimo_ss(Tensor A, Tensor B, Tensor C, Tensor? D, Tensor? zi, Tensor x, bool reverse=False) -> (Tensor, Tensor)",
         {at::Tag::pt2_compliant_tag});
+  m.def("mimo_ss_states(Tensor A, Tensor B, Tensor C, Tensor? D, Tensor? zi, Tensor x, bool reverse=False) -> (Tensor, Tensor, Tensor)",
+        {at::Tag::pt2_compliant_tag});
   m.def("mimo_ss_grad_sums(Tensor? lam, Tensor? hs, Tensor x, Tensor g, int shared, int want, Tensor? Bm=None, "
         "Tensor? Dm=None) -> Tensor[]",
         {at::Tag::pt2_compliant_tag});
@@ -1672,6 +1693,7 @@ TORCH_LIBRARY_IMPL(philtorch, CUDA, m) {
   m.impl("lpv_ss_backward", &lpv_ss_backward_hip);
   m.impl("lpv_ss_states", &lpv_ss_states_hip);
   m.impl("mimo_ss", &mimo_ss_hip);
+  m.impl("mimo_ss_states", &mimo_ss_states_hip);
   m.impl("mimo_ss_grad_sums", &mimo_ss_grad_sums_hip);
   m.impl("lpv_mimo_ss", &lpv_mimo_ss_hip);
   m.impl("lpv_mimo_ss_states", &lpv_mimo_ss_states_hip);

@@ -452,11 +452,18 @@ def _state_space(A, x, B, C, D, zi, unroll_factor, out_idx, fused):
     ops = _mimo_operands(A, x, B, C, D, out_idx, batch, M) if fused and _mimo_applies(
         A, x, B, C, D, zi, unroll_factor) else None
     if ops is not None and ops[0].size(-1) <= 4 and ops[2].size(-2) <= 4:
-        from .. import _op_ctx
+        from .. import _has_op, _op_ctx
 
         x3, Bm, Cm, Dm, vec = ops
+        # A or C with a gradient to come: the forward keeps its states
+        # (mimo_ss_states), which their backward would compute again
+        keep = (torch.is_grad_enabled() and any(t.requires_grad for t in (A, Cm)) and _has_op("mimo_ss_states"))
         with _op_ctx(A, Bm, Cm, Dm, zi, x3):
-            y, zf = torch.ops.philtorch.mimo_ss(A, Bm, Cm, Dm, zi.contiguous() if return_zf else None, x3)
+            args = (A, Bm, Cm, Dm, zi.contiguous() if return_zf else None, x3)
+            if keep:
+                y, zf, _ = torch.ops.philtorch.mimo_ss_states(*args)
+            else:
+                y, zf = torch.ops.philtorch.mimo_ss(*args)
         y = y.squeeze(-1) if vec else y
         return (y, zf) if return_zf else y
     features = -1 if x.dim() == 2 else x.size(-1)
