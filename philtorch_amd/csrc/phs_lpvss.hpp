@@ -153,12 +153,71 @@ __device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X
   }
 }
 
+// The adjoint pass with every gradient of a time-varying biquad (16 x 441000
+// fp32; 68 bytes a step) was bound by its stores: a step's 16-, 8- and 4-byte
+// gradients left lane by lane, 64 separate segments an instruction.  With
+// whole rounds through LDS, b[t] and d[t] read as a lane's vectors and what
+// pass 2 reads issued before the wait for the entry state it took, with its
+// forward, 260 -> 220 us.
+//
+// A round of the wave's lane chunks, scan positions [p0, p0 + 64 K), to the
+// row: where a lane's chunk is more than one 16-byte vector and the round
+// lies inside the row, through the wave's LDS buffer `wb` (lds_flush: 1 KB of
+// the row an instruction), else a lane's own vectors.
+// NB: the buffer's vectors a lane.
+template <bool REV, int NB, typename X, int K>
+__device__ __forceinline__ void lpv_store_round(X *row, int64_t p0, int64_t T, int lane, const X (&v)[K], uint4 *wb) {
+  if constexpr (kLdsBlocked<X, K>) {
+    static_assert(K * int(sizeof(X)) / 16 <= NB, "the round fits the wave's buffer");
+    if (p0 + 64 * K <= T) {
+      constexpr int NV = int(K * sizeof(X) / 16);
+      if constexpr (REV) {
+        X r[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) r[k] = v[K - 1 - k];
+        lds_put_chunk<X, K>(wb, 63 - lane, r);
+      } else {
+        lds_put_chunk<X, K>(wb, lane, v);
+      }
+      lds_flush<NV>(row + (REV ? T - p0 - 64 * K : p0), wb, lane, true);
+      return;
+    }
+  }
+  lpv_store<REV, X, K>(row, p0 + int64_t(lane) * K, T, v);
+}
+
 // Time of scan position s (clamped into the row: positions past it carry a
 // zero input and coefficient, and their outputs are not stored).
 template <bool REV>
 __device__ __forceinline__ int64_t lpv_time(int64_t s, int64_t T) {
   const int64_t t = REV ? T - 1 - s : s;
   return t < 0 ? 0 : (t >= T ? T - 1 : t);
+}
+
+// K steps of an operand from scan position s0: one that lies step by step in
+// memory (a stride of its own size) as a lane's vectors, one constant in time
+// or otherwise strided step by step.  Positions past the row carry a zero
+// input, so what they read does not matter.
+template <bool REV, typename X, int K, typename E>
+__device__ __forceinline__ void lpv_operand(const LpvOperand<E> &o, int64_t b, int64_t s0, int64_t T, X (&out)[K]) {
+  constexpr int N = int(sizeof(X) / sizeof(E));
+  const E *p = o.p + b * o.row_stride;
+  // (one uniform branch for the chunk, none per step)
+  if (o.t_stride == N) {
+    lpv_load<REV, X, K>(reinterpret_cast<const X *>(p), s0, T, out, X{});
+  } else {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      union {
+        X x;
+        E e[N];
+      } u;
+      const E *q = p + lpv_time<REV>(s0 + k, T) * o.t_stride;
+#pragma unroll
+      for (int i = 0; i < N; ++i) u.e[i] = q[i];
+      out[k] = u.x;
+    }
+  }
 }
 
 // b[t] x[t] for the K steps from scan position s0 (b absent: x[t] into
@@ -172,11 +231,18 @@ __device__ __forceinline__ void lpv_inputs(const LpvSsArgs<Alg> &a, int64_t b, i
   // (one uniform branch for the chunk, no per-step select between a load
   // and a constant)
   if (a.bv.p) {
-    const E *bp = a.bv.p + b * a.bv.row_stride;
+    if constexpr (V::M <= 2) {
+      typename Alg::s_state bk[K];
+      lpv_operand<REV, typename Alg::s_state, K>(a.bv, b, s0, a.T_len, bk);
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int64_t t = lpv_time<REV>(s0 + k, a.T_len);
-      X[k] = V::scale(V::load_vec(bp + t * a.bv.t_stride), u[k]);
+      for (int k = 0; k < K; ++k) X[k] = V::scale(bk[k], u[k]);
+    } else {
+      const typename Alg::elem *bp = a.bv.p + b * a.bv.row_stride;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int64_t t = lpv_time<REV>(s0 + k, a.T_len);
+        X[k] = V::scale(V::load_vec(bp + t * a.bv.t_stride), u[k]);
+      }
     }
   } else {
     const typename Alg::s_state e = V::unit(in_idx);
@@ -185,44 +251,40 @@ __device__ __forceinline__ void lpv_inputs(const LpvSsArgs<Alg> &a, int64_t b, i
   }
 }
 
-// One step of the adjoint pass's coefficient gradients at time t of row b
-// (valid: t inside the row): lambda = dL/dh[t+1] (the adjoint state before
-// the step), g = dL/dy[t], hf = h[t], xf = x[t].
+// One step of the adjoint pass's coefficient gradients: lambda = dL/dh[t+1]
+// (the adjoint state before the step), g = dL/dy[t], hf = h[t], xf = x[t].
+// The products of the operands that vary along time go to gA, gb, gc, gd
+// (stored by the caller), those of the others are summed.
 template <class Alg>
-__device__ __forceinline__ void lpv_grad_step(const LpvSsArgs<Alg> &a, int64_t b, int64_t t, bool valid,
-                                              const typename Alg::s_state &lambda, typename Alg::elem g,
-                                              const typename Alg::s_state &hf, typename Alg::elem xf,
-                                              SsGrad<Alg, typename Alg::elem> &acc) {
+__device__ __forceinline__ void lpv_grad_step(const LpvSsArgs<Alg> &a, const typename Alg::s_state &lambda,
+                                              typename Alg::elem g, const typename Alg::s_state &hf,
+                                              typename Alg::elem xf, typename Alg::s_coef &gA,
+                                              typename Alg::s_state &gb, typename Alg::s_state &gc,
+                                              typename Alg::elem &gd, SsGrad<Alg, typename Alg::elem> &acc) {
   using E = typename Alg::elem;
   using G = SsGrad<Alg, E>;
   constexpr int M = G::M;
-  union {
+  union VU {
     typename Alg::s_state s;
     E e[M];
-  } ul, uh;
+  } ul, uh, ub, uc;
   ul.s = lambda;
   uh.s = hf;
-  const int64_t rt = b * a.T_len + t;
-  if (valid && a.gA_step) {
-    union {
-      typename Alg::s_coef s;
-      E e[M * M];
-    } u;
+  union {
+    typename Alg::s_coef s;
+    E e[M * M];
+  } ua;
 #pragma unroll
-    for (int i = 0; i < M; ++i)
+  for (int i = 0; i < M; ++i) {
 #pragma unroll
-      for (int j = 0; j < M; ++j) u.e[i * M + j] = a.gA_trans ? uh.e[i] * ul.e[j] : ul.e[i] * uh.e[j];
-    reinterpret_cast<typename Alg::s_coef *>(a.gA_step)[rt] = u.s;
+    for (int j = 0; j < M; ++j) ua.e[i * M + j] = a.gA_trans ? uh.e[i] * ul.e[j] : ul.e[i] * uh.e[j];
+    ub.e[i] = ul.e[i] * xf;
+    uc.e[i] = g * uh.e[i];
   }
-  if (valid && a.gb_step) {
-#pragma unroll
-    for (int i = 0; i < M; ++i) a.gb_step[rt * M + i] = ul.e[i] * xf;
-  }
-  if (valid && a.gc_step) {
-#pragma unroll
-    for (int i = 0; i < M; ++i) a.gc_step[rt * M + i] = g * uh.e[i];
-  }
-  if (valid && a.gd_step) a.gd_step[rt] = g * xf;
+  gA = ua.s;
+  gb = ub.s;
+  gc = uc.s;
+  gd = g * xf;
   if (a.sum_b) {
 #pragma unroll
     for (int i = 0; i < M; ++i) acc.v[G::kB + i] = fma(ul.e[i], xf, acc.v[G::kB + i]);
@@ -289,6 +351,16 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
   __shared__ S s_in;
   __shared__ unsigned s_id, s_tag;
   __shared__ uint64_t s_look[St::kLookWords];
+  // whole rounds' states and per-step gradients leave through LDS
+  constexpr bool kStates = MODE == kSsStates || MODE == kSsStatesY;
+  // (orders 1-2; a round of 3 x 3 or 4 x 4 gradients would spill, and each
+  // step's matrix is a run of 36 to 128 bytes already)
+  constexpr bool kRound = V::M <= 2;
+  constexpr int kNVh = ((kStates || (MODE == kSsGrad && kRound)) && kLdsBlocked<SS, K>) ? int(K * sizeof(SS) / 16) : 1;
+  constexpr int kNVa = (MODE == kSsGrad && kRound && kLdsBlocked<SC, K>) ? int(K * sizeof(SC) / 16) : 1;
+  constexpr int kNVe = kLdsBlocked<E, K> ? int(K * sizeof(E) / 16) : 1;  // outputs, per-step dL/dd
+  constexpr int kNVm = kNVa > kNVh ? kNVa : kNVh, kNVb = kNVm > kNVe ? kNVm : kNVe;
+  __shared__ uint4 s_out[kNVb > 1 ? kWaves * 64 * kNVb : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -367,39 +439,90 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
     carry = compose<Alg>(carry, tot);
   }
   if (lane == 0) s_wagg[w] = carry;
+  // what pass 2 reads besides: orders 1-2 issue it before the wait for the
+  // entry state; orders 3-4, with no registers to hold it, step by step
+  const E *cp = a.cv.p ? a.cv.p + b * a.cv.row_stride : nullptr;
+  const E *dp = a.d.p ? a.d.p + b * a.d.row_stride : nullptr;
+  const SS c_fixed = V::unit(a.out_idx);
+  constexpr int kRe = kRound ? R : 1, kKe = kRound ? K : 1;
+  SS Cv[kRe][kKe], Hf[MODE == kSsGrad ? R : 1][MODE == kSsGrad ? K : 1];
+  E Dv[kRe][kKe], Xf[MODE == kSsGrad ? R : 1][MODE == kSsGrad ? K : 1];
+  auto read_fwd = [&](int r) {
+    if constexpr (MODE == kSsGrad) {
+      lpv_load<REV, SS, K>(reinterpret_cast<const SS *>(a.hs_fwd) + b * T, chunk0(r), T, Hf[r], SS{});
+      lpv_load<REV, E, K>(a.x_fwd + b * T, chunk0(r), T, Xf[r], E(0));
+    }
+  };
+  if constexpr (kRound) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      read_fwd(r);
+      if constexpr (MODE != kSsStates) {
+        if (cp) {
+          lpv_operand<REV, SS, K>(a.cv, b, chunk0(r), T, Cv[r]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < K; ++k) Cv[r][k] = c_fixed;
+        }
+        if (dp) {
+          lpv_operand<REV, E, K>(a.d, b, chunk0(r), T, Dv[r]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < K; ++k) Dv[r][k] = E(0);
+        }
+      }
+    }
+  }
   __syncthreads();  // wave aggregates are in s_wagg
   __syncthreads();  // entry state is in s_in
   const S hw = apply<Alg>(s_wpre[w], s_in);
 
   // ---- pass 2: y = c[t] . h + d[t] x[t], then the step
-  const E *cp = a.cv.p ? a.cv.p + b * a.cv.row_stride : nullptr;
-  const E *dp = a.d.p ? a.d.p + b * a.d.row_stride : nullptr;
-  const SS c_fixed = V::unit(a.out_idx);
   SsGrad<Alg, E> lacc;
   if constexpr (MODE == kSsGrad) {
 #pragma unroll
     for (int j = 0; j < SsGrad<Alg>::kN; ++j) lacc.v[j] = E(0);
   }
+  uint4 *wb = s_out + (kNVb > 1 ? w * 64 * kNVb : 0);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const int64_t t0 = chunk0(r);
+    const int64_t t0 = chunk0(r), p0 = seg0 + int64_t(r) * 64 * K;
     SS h = Alg::store_s(apply<Alg>(Ex[r], hw));
-    SS Hf[K];
-    E Xf[K];
-    if constexpr (MODE == kSsGrad) {
-      lpv_load<REV, SS, K>(reinterpret_cast<const SS *>(a.hs_fwd) + b * T, t0, T, Hf, SS{});
-      lpv_load<REV, E, K>(a.x_fwd + b * T, t0, T, Xf, E(0));
-    }
+    if constexpr (!kRound) read_fwd(r);
+    SS Hk[K];  // states mode: the state before every step
     E O[K];
+    constexpr int kG = MODE == kSsGrad && kRound ? K : 1;
+    SC GA[kG];
+    SS GB[kG], GC[kG];
+    E GD[kG];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      const int64_t t = lpv_time<REV>(t0 + k, T);
-      if constexpr (MODE == kSsStates || MODE == kSsStatesY) Hf[k] = h;
+      if constexpr (kStates) Hk[k] = h;
       if constexpr (MODE != kSsStates) {
-        const SS c = cp ? V::load_vec(cp + t * a.cv.t_stride) : c_fixed;
-        const E dv = dp ? dp[t * a.d.t_stride] : E(0);
+        SS c;
+        E dv;
+        if constexpr (kRound) {
+          c = Cv[r][k];
+          dv = Dv[r][k];
+        } else {
+          const int64_t t = lpv_time<REV>(t0 + k, T);
+          c = cp ? V::load_vec(cp + t * a.cv.t_stride) : c_fixed;
+          dv = dp ? dp[t * a.d.t_stride] : E(0);
+        }
         O[k] = fma(dv, U[r][k], V::dot(c, h));
-        if constexpr (MODE == kSsGrad) lpv_grad_step<Alg>(a, b, t, t0 + k < T, h, U[r][k], Hf[k], Xf[k], lacc);
+        if constexpr (MODE == kSsGrad) {
+          const int kk = kRound ? k : 0;
+          lpv_grad_step<Alg>(a, h, U[r][k], Hf[r][k], Xf[r][k], GA[kk], GB[kk], GC[kk], GD[kk], lacc);
+          if constexpr (!kRound) {
+            if (t0 + k < T) {
+              const int64_t rt = b * T + lpv_time<REV>(t0 + k, T);
+              if (a.gA_step) reinterpret_cast<SC *>(a.gA_step)[rt] = GA[0];
+              if (a.gb_step) reinterpret_cast<SS *>(a.gb_step)[rt] = GB[0];
+              if (a.gc_step) reinterpret_cast<SS *>(a.gc_step)[rt] = GC[0];
+              if (a.gd_step) a.gd_step[rt] = GD[0];
+            }
+          }
+        }
       }
       h = Alg::s_affine(A[r][k], h, X[r][k]);
       if (MODE != kSsStates && a.zf && t0 + k == T - 1) {
@@ -412,12 +535,17 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
         for (int i = 0; i < V::M; ++i) a.zf[b * V::M + i] = zu.e[i];
       }
     }
-    if constexpr (MODE == kSsStates || MODE == kSsStatesY)
-      lpv_store<REV, SS, K>(reinterpret_cast<SS *>(a.hs) + b * T, t0, T, Hf);
+    if constexpr (kStates) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.hs) + b * T, p0, T, lane, Hk, wb);
+    if constexpr (MODE == kSsGrad && kRound) {
+      if (a.gA_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SC *>(a.gA_step) + b * T, p0, T, lane, GA, wb);
+      if (a.gb_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.gb_step) + b * T, p0, T, lane, GB, wb);
+      if (a.gc_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.gc_step) + b * T, p0, T, lane, GC, wb);
+      if (a.gd_step) lpv_store_round<REV, kNVb>(a.gd_step + b * T, p0, T, lane, GD, wb);
+    }
     if constexpr (MODE == kSsPlain || MODE == kSsStatesY)
-      lpv_store<REV, E, K>(a.y + b * T, t0, T, O);
+      lpv_store_round<REV, kNVb>(a.y + b * T, p0, T, lane, O, wb);
     else if (MODE == kSsGrad && a.y)
-      lpv_store<REV, E, K>(a.y + b * T, t0, T, O);
+      lpv_store_round<REV, kNVb>(a.y + b * T, p0, T, lane, O, wb);
   }
   if constexpr (MODE == kSsGrad) {
     if (a.gpart) {  // the wave's sums of the operands constant in time
