@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor
 
-from .. import EXTENSION_LOADED
+from .. import EXTENSION_LOADED, _run_scan
 
 
 def _native_ok(a: Tensor, init: Tensor, x: Tensor) -> bool:
@@ -64,8 +64,10 @@ def linear_recurrence(a: Tensor, init: Tensor, x: Tensor, *, unroll_factor: int 
     k = unroll_factor
 
     if k == 1 and _native_ok(a, init, x):
-        dt = torch.promote_types(torch.promote_types(a.dtype, init.dtype), x.dtype)
-        return torch.ops.philtorch.recur(a.to(dt), init.to(dt).expand(batch), x.to(dt))
+        if not (a.dtype == init.dtype == x.dtype):
+            dt = torch.promote_types(torch.promote_types(a.dtype, init.dtype), x.dtype)
+            a, init, x = a.to(dt), init.to(dt), x.to(dt)
+        return _run_scan("recur", a, init if init.size(0) == batch else init.expand(batch), x)
 
     if k == 1 or k >= N:
         return _scalar_recursion_loop(a, init, x)

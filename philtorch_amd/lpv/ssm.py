@@ -20,7 +20,7 @@ import torch.nn.functional as F
 from torch import Tensor
 from torch.autograd import Function
 
-from .. import EXTENSION_LOADED, HELION_LOADED
+from .. import EXTENSION_LOADED, HELION_LOADED, _op_ctx, _plain, _run, _run_scan
 
 
 def extension_backend_indicator(x: Tensor, M: int) -> bool:
@@ -42,9 +42,7 @@ class MatrixRecurrence(Function):
 
     @staticmethod
     def forward(A: Tensor, zi: Tensor, x: Tensor) -> Tensor:
-        if x.size(-1) == 2:
-            return torch.ops.philtorch.recur2(A, zi, x)
-        return torch.ops.philtorch.recurN(A, zi, x)
+        return _run_scan("recur2" if x.size(-1) == 2 else "recurN", A, zi, x)
 
     @staticmethod
     def setup_context(ctx: Any, inputs: tuple, output: Tensor) -> None:
@@ -57,7 +55,8 @@ class MatrixRecurrence(Function):
         A, zi, y = ctx.saved_tensors
         needs = ctx.needs_input_grad
         if not torch.is_grad_enabled():
-            gA, gzi, gx = torch.ops.philtorch.recurN_backward(A, zi, y, grad_y)
+            with _op_ctx():
+                gA, gzi, gx = torch.ops.philtorch.recurN_backward(A, zi, y, grad_y)
             return (gA if needs[0] else None, gzi if needs[1] else None, gx if needs[2] else None)
         AH = A.mT.conj_physical()
         coef = torch.roll(AH, -1, dims=-3).flip(-3)
@@ -112,11 +111,14 @@ def _ext_ss_recur(A: Tensor, zi: Tensor, x: Tensor, *, out_idx: Optional[int] = 
     if M == 1:
         xs = x if x.dim() == 2 else x.squeeze(-1)
         coef = A[..., 0, 0]  # [T] shared or [B, T]
-        y = torch.ops.philtorch.recur(coef, zi.reshape(-1), xs).unsqueeze(-1)
+        y = _run_scan("recur", coef, zi.reshape(-1), xs).unsqueeze(-1)
     else:
         if x.dim() == 2:
             x = _widen(x, M)
-        y = MatrixRecurrence.apply(A, zi, x)
+        if _plain((A, zi, x)):
+            y = _run_scan("recur2" if M == 2 else "recurN", A, zi, x)
+        else:
+            y = MatrixRecurrence.apply(A, zi, x)
     if out_idx is not None and y.dim() == 3:
         y = y[:, :, out_idx]
     return y
@@ -611,34 +613,25 @@ def state_space(
     native = extension_backend_indicator(x, M) and unroll_factor in (None, 1)
     ops = _lpv_siso_operands(x, B, C, D, out_idx, batch, N, M)
     if _fused_lpv_ss_applies(A, x, zi if return_zf else None, ops, native):
-        from .. import _has_op, _op_ctx
+        from .. import _has_op
 
         # a coefficient with a gradient to come: the forward keeps its states
         # (lpv_ss_states), which the coefficient backward would compute again
         keep = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (A, *ops))
-        with _op_ctx(A, *ops, zi, x):
-            args = (A, ops[0], ops[1], ops[2], zi.contiguous() if return_zf else None, x,
-                    0 if out_idx is None else out_idx)
-            if keep and _has_op("lpv_ss_states"):
-                y, zf, _ = torch.ops.philtorch.lpv_ss_states(*args)
-            else:
-                y, zf = torch.ops.philtorch.lpv_ss(*args)
+        y, zf = _run("lpv_ss_states" if keep and _has_op("lpv_ss_states") else "lpv_ss", A, ops[0], ops[1], ops[2],
+                     zi.contiguous() if return_zf else None, x, 0 if out_idx is None else out_idx)[:2]
         return (y, zf) if return_zf else y
     mops = _lpv_mimo_operands(x, B, C, D, out_idx, batch, N, M) if native else None
     if _lpv_mimo_applies(A, x, zi if return_zf else None, mops, native):
-        from .. import _has_op, _op_ctx
+        from .. import _has_op
 
         x3, Bm, Cm, Dm, vec = mops
         # a coefficient with a gradient to come: the forward keeps its states
         # (lpv_mimo_ss_states, where outputs and states fit four planes)
         keep = (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (A, Bm, Cm, Dm))
                 and Cm.size(-2) + M <= 4 and _has_op("lpv_mimo_ss_states"))
-        with _op_ctx(A, Bm, Cm, Dm, zi, x3):
-            args = (A, Bm, Cm, Dm, zi.contiguous() if return_zf else None, x3)
-            if keep:
-                y, zf, _ = torch.ops.philtorch.lpv_mimo_ss_states(*args)
-            else:
-                y, zf = torch.ops.philtorch.lpv_mimo_ss(*args)
+        y, zf = _run("lpv_mimo_ss_states" if keep else "lpv_mimo_ss", A, Bm, Cm, Dm,
+                     zi.contiguous() if return_zf else None, x3)[:2]
         y = y.squeeze(-1) if vec else y
         return (y, zf) if return_zf else y
     Bx = _apply_B(x, B, batch, N, M, features)

@@ -120,10 +120,9 @@ def _fused_biquad(b: Tensor, a: Tensor, x: Tensor, zi: Optional[Tensor]):
 
         y, zf = _BiquadColumns.apply(bt, at, zb, x, b_col, a_col)
     else:
-        from .. import _op_ctx
+        from .. import _run
 
-        with _op_ctx(b, a, zb, x):
-            y, zf, _ = torch.ops.philtorch.biquad(b, a, zb, x)
+        y, zf, _ = _run("biquad", b, a, zb, x)
     return y if zi is None else (y, zf)
 
 
@@ -189,16 +188,12 @@ def _fused_lfilter(b: Tensor, a: Tensor, x: Tensor, zi: Optional[Tensor], form: 
     """lfilter(b, a, x, zi, form) through philtorch::lfilter_ss."""
     M = max(b.size(-1) - 1, a.size(-1))
     zb = None if zi is None else zi.expand(x.size(0), M).contiguous()
-    from .. import _has_op, _op_ctx
+    from .. import _has_op, _run
 
     # b or a with a gradient to come: the forward keeps its states
     # (lfilter_ss_states), which their backward would compute again
     keep = torch.is_grad_enabled() and (b.requires_grad or a.requires_grad) and _has_op("lfilter_ss_states")
-    with _op_ctx(b, a, zb, x):
-        if keep:
-            y, zf, _ = torch.ops.philtorch.lfilter_ss_states(b, a, zb, x, 0 if form == "tdf2" else 1)
-        else:
-            y, zf = torch.ops.philtorch.lfilter_ss(b, a, zb, x, 0 if form == "tdf2" else 1)
+    y, zf = _run("lfilter_ss_states" if keep else "lfilter_ss", b, a, zb, x, 0 if form == "tdf2" else 1)[:2]
     return y if zi is None else (y, zf)
 
 
@@ -307,17 +302,14 @@ def _fused_filtfilt(b: Tensor, a: Tensor, x: Tensor, padmode: Optional[str], edg
     """filtfilt of a filter of order 4 at most through philtorch::filtfilt."""
     x2 = x.reshape(-1, x.size(-1))
     code = _PAD_CODES[padmode] if padmode is not None else 0
-    from .. import _has_op, _op_ctx
+    from .. import _has_op, _run
 
     # b or a with a gradient to come: the forward keeps pass 1's output and
     # both passes' states (filtfilt_states), which their backward would
     # compute again
     keep = torch.is_grad_enabled() and (b.requires_grad or a.requires_grad) and _has_op("filtfilt_states")
-    with _op_ctx(b, a, x2):
-        if keep:
-            y = torch.ops.philtorch.filtfilt_states(b, a, x2, code, edge if padmode is not None else 0)[0]
-        else:
-            y = torch.ops.philtorch.filtfilt(b, a, x2, code, edge if padmode is not None else 0)
+    e = edge if padmode is not None else 0
+    y = _run("filtfilt_states", b, a, x2, code, e)[0] if keep else _run("filtfilt", b, a, x2, code, e)
     return y.reshape(x.shape)
 
 
@@ -413,14 +405,13 @@ def _sosfilt_fused(sos: Tensor, x: Tensor, zi: Optional[Tensor]) -> tuple[Tensor
         zi = None if zi is None else zi.float()
     else:
         sos = sos.to(dtype)
-    from .. import _op_ctx
+    from .. import _run
 
     y, zfs = x, []
     for s0 in range(0, sos.size(-2), _SOS_SECTIONS_PER_CALL):
         part = sos[..., s0:s0 + _SOS_SECTIONS_PER_CALL, :]
         zpart = None if zi is None else zi[:, s0:s0 + part.size(-2)].contiguous()
-        with _op_ctx(part, zpart, y):
-            y, zf, _ = torch.ops.philtorch.sosfilt(part.contiguous(), zpart, y.contiguous())
+        y, zf, _ = _run("sosfilt", part.contiguous(), zpart, y.contiguous())
         zfs.append(zf)
     return y.to(dtype), torch.cat(zfs, dim=1).to(dtype)
 

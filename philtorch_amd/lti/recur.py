@@ -15,6 +15,8 @@ import torch.nn.functional as F
 from torch import Tensor
 from torch.autograd import Function
 
+from .. import _op_ctx, _run_scan
+
 
 class LTIRecurrence(Function):
     """Autograd Function of the native scalar LTI scan.
@@ -31,7 +33,7 @@ class LTIRecurrence(Function):
 
     @staticmethod
     def forward(a: Tensor, init: Tensor, x: Tensor) -> Tensor:
-        return torch.ops.philtorch.lti_recur(a, init, x)
+        return _run_scan("lti_recur", a, init, x)
 
     @staticmethod
     def setup_context(ctx: Any, inputs: tuple, output: Tensor) -> None:
@@ -44,7 +46,8 @@ class LTIRecurrence(Function):
         a, init, out = ctx.saved_tensors
         needs = ctx.needs_input_grad
         if not torch.is_grad_enabled():
-            ga, gi, gx = torch.ops.philtorch.lti_recur_backward(a, init, out, grad_out)
+            with _op_ctx():
+                ga, gi, gx = torch.ops.philtorch.lti_recur_backward(a, init, out, grad_out)
             return (ga if needs[0] else None, gi if needs[1] else None, gx if needs[2] else None)
 
         a_conj = a.conj_physical()

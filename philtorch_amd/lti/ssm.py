@@ -17,7 +17,7 @@ import torch.nn.functional as F
 from torch import Tensor
 from torch.autograd import Function
 
-from .. import EXTENSION_LOADED, HELION_LOADED
+from .. import EXTENSION_LOADED, HELION_LOADED, _op_ctx, _plain, _run, _run_scan
 from .recur import LTIRecurrence, linear_recurrence
 
 
@@ -46,9 +46,7 @@ class LTIMatrixRecurrence(Function):
 
     @staticmethod
     def forward(A: Tensor, zi: Tensor, x: Tensor) -> Tensor:
-        if x.size(-1) == 2:
-            return torch.ops.philtorch.lti_recur2(A, zi, x)
-        return torch.ops.philtorch.lti_recurN(A, zi, x)
+        return _run_scan("lti_recur2" if x.size(-1) == 2 else "lti_recurN", A, zi, x)
 
     @staticmethod
     def setup_context(ctx: Any, inputs: tuple, output: Tensor) -> None:
@@ -61,7 +59,8 @@ class LTIMatrixRecurrence(Function):
         A, zi, y = ctx.saved_tensors
         needs = ctx.needs_input_grad
         if not torch.is_grad_enabled():
-            gA, gzi, gx = torch.ops.philtorch.lti_recurN_backward(A, zi, y, grad_y)
+            with _op_ctx():
+                gA, gzi, gx = torch.ops.philtorch.lti_recurN_backward(A, zi, y, grad_y)
             return (gA if needs[0] else None, gzi if needs[1] else None, gx if needs[2] else None)
         AH = A.mT.conj_physical()
         lam = LTIMatrixRecurrence.apply(AH, torch.zeros_like(zi), grad_y.flip(1)).flip(1)
@@ -113,7 +112,10 @@ def _ext_ss_recur(A: Tensor, zi: Tensor, x: Tensor, *, out_idx: Optional[int] = 
     else:
         if x.dim() == 2:
             x = _widen(x, A.size(-1))
-        y = LTIMatrixRecurrence.apply(A, zi, x)
+        if _plain((A, zi, x)):
+            y = _run_scan("lti_recur2" if A.size(-1) == 2 else "lti_recurN", A, zi, x)
+        else:
+            y = LTIMatrixRecurrence.apply(A, zi, x)
     if out_idx is not None and y.dim() == 3:
         y = y[:, :, out_idx]
     return y
@@ -436,34 +438,26 @@ def _state_space(A, x, B, C, D, zi, unroll_factor, out_idx, fused):
     if unroll_factor is None:
         unroll_factor = round(N**0.5)
     if fused and _fused_ss_applies(A, x, B, C, D, zi, unroll_factor, out_idx):
-        from .. import _has_op, _op_ctx
+        from .. import _has_op
 
         # a coefficient with a gradient to come: the forward keeps its states
         # (lti_ss_states), which the coefficient backward would compute again
         keep = (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (A, B, C, D))
                 and _has_op("lti_ss_states"))
-        with _op_ctx(A, B, C, D, zi, x):
-            args = (A, B, C, D, zi.contiguous() if return_zf else None, x, out_idx if C is None else 0)
-            if keep:
-                y, zf, _ = torch.ops.philtorch.lti_ss_states(*args)
-            else:
-                y, zf = torch.ops.philtorch.lti_ss(*args)
+        y, zf = _run("lti_ss_states" if keep else "lti_ss", A, B, C, D, zi.contiguous() if return_zf else None, x,
+                     out_idx if C is None else 0)[:2]
         return (y, zf) if return_zf else y
     ops = _mimo_operands(A, x, B, C, D, out_idx, batch, M) if fused and _mimo_applies(
         A, x, B, C, D, zi, unroll_factor) else None
     if ops is not None and ops[0].size(-1) <= 4 and ops[2].size(-2) <= 4:
-        from .. import _has_op, _op_ctx
+        from .. import _has_op
 
         x3, Bm, Cm, Dm, vec = ops
         # A or C with a gradient to come: the forward keeps its states
         # (mimo_ss_states), which their backward would compute again
         keep = (torch.is_grad_enabled() and any(t.requires_grad for t in (A, Cm)) and _has_op("mimo_ss_states"))
-        with _op_ctx(A, Bm, Cm, Dm, zi, x3):
-            args = (A, Bm, Cm, Dm, zi.contiguous() if return_zf else None, x3)
-            if keep:
-                y, zf, _ = torch.ops.philtorch.mimo_ss_states(*args)
-            else:
-                y, zf = torch.ops.philtorch.mimo_ss(*args)
+        y, zf = _run("mimo_ss_states" if keep else "mimo_ss", A, Bm, Cm, Dm, zi.contiguous() if return_zf else None,
+                     x3)[:2]
         y = y.squeeze(-1) if vec else y
         return (y, zf) if return_zf else y
     features = -1 if x.dim() == 2 else x.size(-1)
