@@ -128,6 +128,13 @@ Layout make_layout(int64_t B, int64_t T, bool TV, bool shared, bool backward) {
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Whether a launch that writes step_bytes per step and row stores past the
+// caches (what fp32 elements always do; see kStreamAlways).
+constexpr double kStreamedBytes = 134217728.0;
+inline bool streams_out(int64_t B, int64_t T, size_t step_bytes) {
+  return double(B) * double(T) * double(step_bytes) >= kStreamedBytes;
+}
+
 // Tile id -> row by multiply and shift (the kernels' `id / B` without a
 // 64-bit division): with l = ceil(log2 B) and s = 31 + l, m = floor(2^s / B)
 // + 1 gives floor(id m / 2^s) = floor(id / B) for every id below 2^31
@@ -209,6 +216,9 @@ int launch(int64_t B, int64_t T, bool TV, bool shared, bool backward, const void
   a.spin_limit = sl ? sl : kDefaultSpinLimit;
   a.agg_only = g_agg_only.load(std::memory_order_relaxed) ? 1u : 0u;
   row_split(B, a.b_magic, a.b_shift);
+  const bool step_grads = backward && TV && gcoef;
+  a.streamed = streams_out(B, T, (out ? sizeof(typename Alg::s_state) : 0) +
+                                     (step_grads ? sizeof(typename Alg::s_coef) : 0));
   a.trace = nullptr;
   a.trace_tiles = 0;
   if (backward && gcoef) {

@@ -123,6 +123,7 @@ struct ScanArgs {
   unsigned per_stripe;         // claims per stripe (grid = per_stripe * kStripes)
   unsigned spin_limit;         // look-back polls before the self-compute fallback
   unsigned agg_only;           // testing: tiles after a row's first publish no inclusive state
+  bool streamed;               // outputs leave past the caches (streams_out)
   // tile id -> (scan position, row) without a 64-bit division: for ids
   // below 2^31, id / B == (id * b_magic) >> b_shift (set by the host)
   uint64_t b_magic;
@@ -262,6 +263,35 @@ struct __attribute__((packed, aligned(4))) RowVec {
 };
 __device__ __forceinline__ RowVec row_vec(const uint4 &v) { return {v.x, v.y, v.z, v.w}; }
 
+// Stores past the caches.  The scans write every output once and are bound
+// by memory; a plain store's line stays in an L2 until it is written back
+// (at the latest as the launch ends) and takes the place of lines another
+// launch could read.  Kernel time, forward + backward, plain / streamed (us),
+// 16 fp32 rows: scalar scan of 131072 steps 19.6 / 18.0, 524288 58.8 / 56.6,
+// 2097152 232 / 220; 2x2 scan of 32768 23.7 / 22.5, 262144 100.4 / 93.3; the
+// time-varying biquad of 16384 23.2 / 23.4, 65536 39.4 / 37.0, 262144
+// 141.6 / 132.  With 8-byte elements the forward gains and a backward that
+// finds y in the 256 MB last-level cache may lose more: 64 fp64 rows of 32768
+// 27.8 / 28.5, 64 complex64 LTI rows of 32768 32.9 / 30.6, 65536
+// 45.8 / 46.2, 98304 65.8 / 61.1, 131072 86.6 / 88.0, 196608 124 / 126.3; from
+// 128 MB of outputs on, which with their inputs fill that cache, it only
+// gains: 262144 172 / 167.6, 524288 325 / 309.  So fp32 elements always
+// stream and wider ones from 128 MB on (streams_out in the launch code).
+// Kernels whose outputs the same call reads next (the cascades, filtfilt:
+// 40.7 / 43.1) store plainly.
+template <typename E>
+constexpr bool kStreamAlways = std::is_same<E, float>::value;
+
+// The empty statements keep this store and a plain one on the two sides of a
+// branch apart: merged, they lose the mark.
+__device__ __forceinline__ void store_streamed(RowVec *p, const RowVec &v) {
+  typedef uint32_t Words __attribute__((ext_vector_type(4), aligned(4)));
+  const Words t = {v.x, v.y, v.z, v.w};
+  asm volatile("");
+  __builtin_nontemporal_store(t, reinterpret_cast<Words *>(p));
+  asm volatile("");
+}
+
 // ------------------------------------------------------------ coalesced stores
 // A lane that owns K consecutive steps writes them as NV 16-byte vectors of
 // its own, so one store instruction of the wave touches 64 separate
@@ -301,14 +331,18 @@ __device__ __forceinline__ void lds_put_chunk(uint4 *wb, int L, const X (&v)[K])
 // The wave's buffer to its block at dst (in range): vector c of the block is
 // block lane c / NV's vector c % NV.
 template <int NV>
-__device__ __forceinline__ void lds_flush(void *dst, const uint4 *wb, int lane, bool write) {
+__device__ __forceinline__ void lds_flush(void *dst, const uint4 *wb, int lane, bool write, bool streamed = false) {
   wave_sync();
   if (write) {
     RowVec *out = static_cast<RowVec *>(dst);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int c = j * 64 + lane, L = c / NV, v = c % NV;
-      out[c] = row_vec(wb[L * NV + (v ^ lds_swizzle<NV>(L))]);
+      const RowVec u = row_vec(wb[L * NV + (v ^ lds_swizzle<NV>(L))]);
+      if (streamed)
+        store_streamed(out + c, u);
+      else
+        out[c] = u;
     }
   }
   wave_sync();  // later writes to the buffer follow these reads
@@ -468,7 +502,8 @@ __device__ __forceinline__ void load_chunk(const X *row, int64_t t0, int64_t T, 
 }
 
 template <typename X, int K, bool kFull = false>
-__device__ __forceinline__ void store_chunk(X *row, int64_t t0, int64_t T, const X (&v)[K]) {
+__device__ __forceinline__ void store_chunk(X *row, int64_t t0, int64_t T, const X (&v)[K],
+                                            bool streamed = false) {
   if (kFull || t0 + K <= T) {
     constexpr int nv = int(K * sizeof(X) / 16);
     union {
@@ -479,7 +514,12 @@ __device__ __forceinline__ void store_chunk(X *row, int64_t t0, int64_t T, const
     for (int k = 0; k < K; ++k) u.x[k] = v[k];
     RowVec *p = reinterpret_cast<RowVec *>(row + t0);
 #pragma unroll
-    for (int i = 0; i < nv; ++i) p[i] = u.v[i];
+    for (int i = 0; i < nv; ++i) {
+      if (streamed)
+        store_streamed(p + i, u.v[i]);
+      else
+        p[i] = u.v[i];
+    }
   } else {
 #pragma unroll
     for (int k = 0; k < K; ++k)
@@ -825,6 +865,7 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
       const int64_t blk0 = t0 - int64_t(pl) * K;
       const bool blk_full = kFull || blk0 + 64 * K <= T;
       uint4 *wb = s_out + w * 64 * kNVb;
+      const bool streamed = kStreamAlways<typename Alg::elem> || a.streamed;
       if constexpr (!REV) {
         SS O[K];
 #pragma unroll
@@ -835,10 +876,10 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
         if (kSLds && blk_full) {
           if constexpr (kSLds) {
             lds_put_chunk<SS, K>(wb, pl, O);
-            lds_flush<kNVs>(yrow + blk0, wb, lane, true);
+            lds_flush<kNVs>(yrow + blk0, wb, lane, true, streamed);
           }
         } else {
-          store_chunk<SS, K, kFull>(yrow, t0, T, O);
+          store_chunk<SS, K, kFull>(yrow, t0, T, O, streamed);
         }
       } else {
         SS nu = h;
@@ -861,19 +902,19 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
         if (kSLds && blk_full) {
           if constexpr (kSLds) {
             lds_put_chunk<SS, K>(wb, pl, GX);
-            lds_flush<kNVs>(gxrow + blk0, wb, lane, gxrow != nullptr);
+            lds_flush<kNVs>(gxrow + blk0, wb, lane, gxrow != nullptr, streamed);
           }
         } else if (gxrow) {
-          store_chunk<SS, K, kFull>(gxrow, t0, T, GX);
+          store_chunk<SS, K, kFull>(gxrow, t0, T, GX, streamed);
         }
         if constexpr (TV) {
           if (kCLds && blk_full) {
             if constexpr (kCLds) {
               lds_put_chunk<SC, K>(wb, pl, GC);
-              lds_flush<kNVc>(gcrow + blk0, wb, lane, gcrow != nullptr);
+              lds_flush<kNVc>(gcrow + blk0, wb, lane, gcrow != nullptr, streamed);
             }
           } else if (gcrow) {
-            store_chunk<SC, K, kFull>(gcrow, t0, T, GC);
+            store_chunk<SC, K, kFull>(gcrow, t0, T, GC, streamed);
           }
         }
       }
