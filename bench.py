@@ -29,7 +29,7 @@ adjoint op (grads w.r.t. the coefficients, the input and the initial state):
                     philtorch::lfilter_ss_backward given its states)
   c4_mimo  lti.state_space of order 4, 2 inputs and 2 outputs per step (philtorch::mimo_ss)
   c4_mimo_grad  the same plus gradients w.r.t. x and zi (the adjoint mimo_ss pass)
-  c4_mimo_coef  the same plus gradients w.r.t. A, B, C, D (two states passes and the fused sums)
+  c4_mimo_coef  the same plus gradients w.r.t. A, B, C, D (the adjoint-states pass and the fused sums)
   c3_lpv_mimo  lpv.state_space on C3's A[t], 2 inputs and 2 outputs per step (philtorch::lpv_mimo_ss)
   c3_lpv_mimo_grad  the same plus gradients w.r.t. x and zi; c3_lpv_mimo_coef: and A[t], B, C, D
 --composed runs an API config (c3_lpv_ss*, c3_lpv_mimo*, c4_api, c4_lfilter*, c4_filtfilt*, c4_mimo*)
@@ -870,9 +870,9 @@ class MimoSsGrad(MimoSsApi):
 
 class MimoSsCoefGrad(MimoSsGrad):
     """c4_mimo_coef: c4_mimo_grad with the gradients of A, B, C and D too:
-    the forward again writing its states (C = I), the adjoint writing its
-    states (which also gives grad_zi), and one philtorch::mimo_ss_grad_sums
-    pass that sums the four products over time (and rows, for the shared B,
+    the forward keeps its states (philtorch::mimo_ss_states), the adjoint
+    writes its states (which also gives grad_zi), and one
+    philtorch::mimo_ss_grad_sums pass that sums the four products over time (and rows, for the shared B,
     C, D) and writes grad_x = B^T lambda + D^T g."""
 
     def __init__(self):
@@ -881,10 +881,11 @@ class MimoSsCoefGrad(MimoSsGrad):
         self.name = "c4_mimo_coef"
         self.metric = (f"GSamples/s fwd+bwd(x, zi, A, B, C, D), lti.state_space order {M}, {F} inputs, {P} outputs "
                        f"per step B={B} T={T} fp32 (API)")
-        # states (read x, write h), adjoint states (read g, write lambda), then the sums pass (read
-        # lambda, h, x, g; write grad_x)
-        self.bwd_bytes = 4 * ((F + M) + (P + M) + (M + M + F + P + F)) * B * T
-        self.bwd_launch_bytes = 4 * (F + M) * B * T  # the states pass
+        # the forward also writes its states; backward: adjoint states (read g, write lambda), then the
+        # sums pass (read lambda, h, x, g; write grad_x)
+        self.fwd_bytes += 4 * M * B * T
+        self.bwd_bytes = 4 * ((P + M) + (M + M + F + P + F)) * B * T
+        self.bwd_launch_bytes = 4 * (P + M) * B * T  # the adjoint-states pass
 
     def step_fwd(self):
         from philtorch_amd import lti

@@ -155,7 +155,7 @@ __device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X
 }
 
 // The adjoint pass with every gradient of a time-varying biquad (16 x 441000
-// fp32; 68 bytes a step) was bound by its stores: a step's 16-, 8- and 4-byte
+// fp32; 76 bytes a step) was bound by its stores: a step's 16-, 8- and 4-byte
 // gradients left lane by lane, 64 separate segments an instruction.  With
 // whole rounds through LDS, b[t] and d[t] read as a lane's vectors and what
 // pass 2 reads issued before the wait for the entry state it took, with its
