@@ -226,9 +226,13 @@ def _plain(tensors) -> bool:
     """Whether an eager call on these tensors sees no transform that has to
     find the op itself: no functorch level, torch.compile or jit trace, no
     dispatch or function mode, no forward-mode AD level, no tensor subclass."""
+    # first and by itself: dynamo folds it to a constant, and cannot trace the
+    # questions below (it would break the graph here, or refuse fullgraph)
+    if torch.compiler.is_compiling():
+        return False
     return (fwAD._current_level < 0 and not torch._C._are_functorch_transforms_active()
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
-            and not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
+            and torch._C._get_tracing_state() is None
             and all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors))
 
 

@@ -119,3 +119,87 @@ def test_functorch_grad_and_modes_reach_the_op():
     assert pa._plain((a, torch.nn.Parameter(z)))
     y = torch.compile(lambda v: lpv.linear_recurrence(a, z, v, unroll_factor=1), backend="aot_eager")(v)
     assert torch.allclose(y, lpv.linear_recurrence(a, z, u, unroll_factor=1))
+
+
+def _whole_graph_cases():
+    """name -> (call, arguments, the op the captured graph has to hold).  The matrix scans and
+    LTIRecurrence have a jvp of their own, which dynamo refuses where a gradient is recorded."""
+    g = torch.Generator().manual_seed(3)
+    r = lambda *s: torch.rand(*s, generator=g) - 0.5  # noqa: E731
+    B, T, M = 3, 9, 2
+    return {
+        "lpv.linear_recurrence": (lambda a, z, x: lpv.linear_recurrence(a, z, x, unroll_factor=1),
+                                  (r(B, T), r(B), r(B, T)), "recur"),
+        "LTIRecurrence": (lti.LTIRecurrence.apply, (r(B), r(B), r(B, T)), "lti_recur"),
+        "lpv.state_space_recursion": (lambda A, z, x: lpv.state_space_recursion(A, z, x, unroll_factor=1),
+                                      (r(B, T, M, M), r(B, M), r(B, T, M)), "recur2"),
+        "lti.state_space_recursion": (lambda A, z, x: lti.state_space_recursion(A, z, x, unroll_factor=1),
+                                      (r(B, 3, 3), r(B, 3), r(B, T, 3)), "lti_recurN"),
+        "lti.lfilter": (lambda b, a, x: lti.lfilter(b, a, x, unroll_factor=1), (r(B, 3), r(B, 2), r(B, T)),
+                        "lti_recur2"),
+        "lti.filtfilt": (lambda b, a, x: lti.filtfilt(b, a, x, padlen=3, unroll_factor=1),
+                         (r(B, 3), r(B, 2), r(B, T)), "lti_recur2"),
+    }
+
+
+@pytest.mark.parametrize("grad,name", [(False, n) for n in _whole_graph_cases()] + [(True, "lpv.linear_recurrence")])
+def test_compiles_whole(grad, name):
+    f, args, op = _whole_graph_cases()[name]
+    args = [t.clone().requires_grad_(grad) for t in args]
+    seen = []
+
+    def backend(gm, example):
+        seen.extend(str(n.target) for n in gm.graph.nodes)
+        return gm.forward
+
+    torch._dynamo.reset()
+    y = torch.compile(lambda *t: f(*t), fullgraph=True, backend=backend)(*args)
+    assert any(f"philtorch.{op}" in s for s in seen)
+    want = f(*args)
+    assert torch.allclose(y, want, rtol=1e-5, atol=1e-6)  # the same kernel on the same inputs
+    if grad:
+        for p, q in zip(torch.autograd.grad(y.sum(), args), torch.autograd.grad(want.sum(), args)):
+            assert torch.allclose(p, q, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("name", ["_fused_lfilter", "_fused_biquad", "_fused_filtfilt", "_sosfilt_fused"])
+def test_fused_routes_are_captured_whole(name):
+    """The routes of HIP tensors, where a gradient is recorded: what dynamo hands its backend (their
+    kernels take no CPU tensors, so the graph is looked at and not run)."""
+    from philtorch_amd.lti import filtering
+
+    g = torch.Generator().manual_seed(3)
+    r = lambda *s: (torch.rand(*s, generator=g) - 0.5).requires_grad_(True)  # noqa: E731
+    b, a, x = r(3, 3), r(3, 2), r(3, 9)
+    sos = torch.cat([torch.rand(3, 2, 3), torch.ones(3, 2, 1), torch.rand(3, 2, 2) / 4], -1).requires_grad_(True)
+    f, args, op = {
+        "_fused_lfilter": (lambda b, a, x: filtering._fused_lfilter(b, a, x, None, "tdf2"), (b, a, x),
+                           "lfilter_ss_states"),
+        "_fused_biquad": (lambda b, a, x: filtering._fused_biquad(b, a, x, None), (b, a, x), "biquad"),
+        "_fused_filtfilt": (lambda b, a, x: filtering._fused_filtfilt(b, a, x, None, 0), (b, a, x),
+                            "filtfilt_states"),
+        "_sosfilt_fused": (lambda s, x: filtering._sosfilt_fused(s, x, None)[0], (sos, x), "sosfilt"),
+    }[name]
+    seen = []
+
+    def backend(gm, example):
+        seen.extend(str(n.target) for n in gm.graph.nodes)
+        raise RuntimeError("seen")
+
+    torch._dynamo.reset()
+    with pytest.raises(Exception, match="seen"):
+        torch.compile(f, fullgraph=True, backend=backend)(*args)
+    assert any(f"philtorch.{op}" in s for s in seen)
+
+
+@pytest.mark.parametrize("name", list(_whole_graph_cases()))
+def test_exports_strictly(name):
+    f, args, op = _whole_graph_cases()[name]
+
+    class Mod(torch.nn.Module):
+        def forward(self, *t):
+            return f(*t)
+
+    ep = torch.export.export(Mod(), args, strict=True)
+    assert any(f"philtorch.{op}" in str(n.target) for n in ep.graph.nodes)
+    assert torch.allclose(ep.module()(*args), f(*args), rtol=1e-5, atol=1e-6)
