@@ -128,11 +128,29 @@ Layout make_layout(int64_t B, int64_t T, bool TV, bool shared, bool backward) {
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Whether a launch that writes step_bytes per step and row stores past the
-// caches (what fp32 elements always do; see kStreamAlways).
-constexpr double kStreamedBytes = 134217728.0;
-inline bool streams_out(int64_t B, int64_t T, size_t step_bytes) {
-  return double(B) * double(T) * double(step_bytes) >= kStreamedBytes;
+// Whether a scan that writes out (out_step bytes a step and row) and gcoef
+// (gcoef_step) stores past the caches, where kStreams says it can: from 1 GiB
+// of outputs on, with rows of whole 128-byte lines.  One launch each, plain /
+// streamed (us), the step being the forward and its backward at once:
+//   fp32 LPV scan, 1024 x 262144 forward 600 / 586, backward 1020 / 1009, step
+//     1625 / 1589; 8 x 2^24 step 901 / 894
+//   fp64 LPV scan, 8 x 2^24 step 1839 / 1804; 2048 x 65536 step 1650 / 1609
+//   complex64 LTI backward, 1024 x 262144 1278 / 1251
+//   2x2 fp64 LPV scan, 64 x 2^20 step 3047 / 2977
+// Below, what the step gains a launch by itself loses, and more at smaller
+// sizes: fp32, 1024 x 16384 backward 61.7 / 66.8, step 98.7 / 94.3; complex64
+// LTI, 1024 x 16384 step 128 / 133; fp32, 64 x 65536 backward with y still
+// cached 14.7 / 16.6, step 32.2 / 34.0.  Rows that start inside a line lose at
+// any size, as their vectors write it in parts: fp64, 32 x 3000001 step 1204 /
+// 1251.
+constexpr double kStreamedBytes = 1073741824.0;
+inline bool streams_out(int64_t B, int64_t T, const void *out, size_t out_step, const void *gcoef,
+                        size_t gcoef_step) {
+  auto lines = [&](const void *p, size_t step) {
+    return !p || (reinterpret_cast<uintptr_t>(p) % 128 == 0 && size_t(T) * step % 128 == 0);
+  };
+  const double bytes = double((out ? out_step : 0) + (gcoef ? gcoef_step : 0)) * double(B) * double(T);
+  return bytes >= kStreamedBytes && lines(out, out_step) && lines(gcoef, gcoef_step);
 }
 
 // Tile id -> row by multiply and shift (the kernels' `id / B` without a
@@ -178,6 +196,12 @@ void launch_scan(ScanArgs<Alg> a, unsigned grid, hipStream_t stream) {
       return;
     }
   }
+  if constexpr (kStreams<Alg, TV, REV>) {
+    if (streams_out(a.B, a.T_len, a.out, sizeof(typename Alg::s_state), a.gcoef, sizeof(typename Alg::s_coef))) {
+      launch_kernel(scan_kernel<Alg, TV, REV, false, true>, dim3(grid), dim3(Shape<Alg, TV>::kThreads), 0, stream, a);
+      return;
+    }
+  }
   launch_kernel(scan_kernel<Alg, TV, REV>, dim3(grid), dim3(Shape<Alg, TV>::kThreads), 0, stream, a);
 }
 
@@ -216,9 +240,6 @@ int launch(int64_t B, int64_t T, bool TV, bool shared, bool backward, const void
   a.spin_limit = sl ? sl : kDefaultSpinLimit;
   a.agg_only = g_agg_only.load(std::memory_order_relaxed) ? 1u : 0u;
   row_split(B, a.b_magic, a.b_shift);
-  const bool step_grads = backward && TV && gcoef;
-  a.streamed = streams_out(B, T, (out ? sizeof(typename Alg::s_state) : 0) +
-                                     (step_grads ? sizeof(typename Alg::s_coef) : 0));
   a.trace = nullptr;
   a.trace_tiles = 0;
   if (backward && gcoef) {

@@ -82,7 +82,6 @@ int lpv_ss_fwd(int64_t B, int64_t T, const void *A, bool A_sh, bool A_tr, LpvOpe
   if (double(B) * double(tiles_per_row) >= 2147483648.0) return PHS_ERR_INVALID;
   if (!workspace || ws_bytes < lpv_ss_ws_bytes<Alg>(B, T)) return PHS_ERR_WORKSPACE;
   LpvSsArgs<Alg> a = lpv_args<Alg>(B, T, A, A_sh, A_tr, bv, cv, out_idx, 0, d, zi, x, y, zf, workspace);
-  a.streamed = streams_out(B, T, (hs ? M + 1 : 1) * sizeof(E));
   if (hs) {
     a.hs = static_cast<E *>(hs);
     return rev ? lpv_launch<Alg, true, kSsStatesY>(a, stream) : lpv_launch<Alg, false, kSsStatesY>(a, stream);
@@ -175,7 +174,6 @@ int lpv_ss_bwd(int64_t B, int64_t T, const void *A, bool A_sh, bool A_tr, LpvOpe
   if (T > 0) {
     LpvSsArgs<Alg> p = lpv_args<Alg>(B, T, A, A_sh, A_tr, bv, cv, out_idx, 0, d, zi, x, nullptr, nullptr, workspace);
     p.hs = states;
-    p.streamed = streams_out(B, T, M * sizeof(E));
     int rc = PHS_OK;
     if (!hs_in) {
       rc = rev ? lpv_launch<Alg, true, kSsStates>(p, stream) : lpv_launch<Alg, false, kSsStates>(p, stream);
@@ -191,10 +189,6 @@ int lpv_ss_bwd(int64_t B, int64_t T, const void *A, bool A_sh, bool A_tr, LpvOpe
     q.gd_step = step_dst[3];
     q.gA_trans = A_tr ? 1 : 0;
     q.sum_b = sum_b, q.sum_c = sum_c, q.sum_d = sum_d;
-    size_t step_bytes = sizeof(E);  // gx, and the gradients along time
-    for (int i = 0; i < 4; ++i)
-      if (step_dst[i]) step_bytes += (i == 0 ? M * M : i == 3 ? 1 : M) * sizeof(E);
-    q.streamed = streams_out(B, T, step_bytes);
     q.gpart = (sum_b || sum_c || sum_d) ? gpart : nullptr;
     rc = rev ? lpv_launch<Alg, false, kSsGrad>(q, stream) : lpv_launch<Alg, true, kSsGrad>(q, stream);
     if (rc != PHS_OK) return rc;

@@ -69,7 +69,6 @@ struct LpvSsArgs {
   unsigned long long *claims;
   unsigned tiles, per_stripe, spin_limit;
   unsigned agg_only;  // testing: tiles after a row's first publish no inclusive state
-  bool streamed;      // outputs leave past the caches (streams_out)
   uint64_t *status;
 };
 
@@ -127,11 +126,11 @@ __device__ __forceinline__ void lpv_load(const X *row, int64_t s0, int64_t T, X 
 }
 
 template <bool REV, typename X, int K>
-__device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X (&v)[K], bool streamed) {
+__device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X (&v)[K]) {
   constexpr bool kVec = (K * sizeof(X)) % 16 == 0;
   if constexpr (!REV) {
     if constexpr (kVec) {
-      store_chunk<X, K>(row, s0, T, v, streamed);
+      store_chunk<X, K>(row, s0, T, v);
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k)
@@ -143,7 +142,7 @@ __device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X
       X tmp[K];
 #pragma unroll
       for (int k = 0; k < K; ++k) tmp[k] = v[K - 1 - k];
-      if constexpr (kVec) store_chunk<X, K>(row, base, T, tmp, streamed);
+      if constexpr (kVec) store_chunk<X, K>(row, base, T, tmp);
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
@@ -167,8 +166,7 @@ __device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X
 // the row an instruction), else a lane's own vectors.
 // NB: the buffer's vectors a lane.
 template <bool REV, int NB, typename X, int K>
-__device__ __forceinline__ void lpv_store_round(X *row, int64_t p0, int64_t T, int lane, const X (&v)[K], uint4 *wb,
-                                                bool streamed) {
+__device__ __forceinline__ void lpv_store_round(X *row, int64_t p0, int64_t T, int lane, const X (&v)[K], uint4 *wb) {
   if constexpr (kLdsBlocked<X, K>) {
     static_assert(K * int(sizeof(X)) / 16 <= NB, "the round fits the wave's buffer");
     if (p0 + 64 * K <= T) {
@@ -181,11 +179,11 @@ __device__ __forceinline__ void lpv_store_round(X *row, int64_t p0, int64_t T, i
       } else {
         lds_put_chunk<X, K>(wb, lane, v);
       }
-      lds_flush<NV>(row + (REV ? T - p0 - 64 * K : p0), wb, lane, true, streamed);
+      lds_flush<NV>(row + (REV ? T - p0 - 64 * K : p0), wb, lane, true);
       return;
     }
   }
-  lpv_store<REV, X, K>(row, p0 + int64_t(lane) * K, T, v, streamed);
+  lpv_store<REV, X, K>(row, p0 + int64_t(lane) * K, T, v);
 }
 
 // Time of scan position s (clamped into the row: positions past it carry a
@@ -486,7 +484,6 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
     for (int j = 0; j < SsGrad<Alg>::kN; ++j) lacc.v[j] = E(0);
   }
   uint4 *wb = s_out + (kNVb > 1 ? w * 64 * kNVb : 0);
-  const bool streamed = kStreamAlways<E> || a.streamed;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int64_t t0 = chunk0(r), p0 = seg0 + int64_t(r) * 64 * K;
@@ -538,17 +535,17 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
         for (int i = 0; i < V::M; ++i) a.zf[b * V::M + i] = zu.e[i];
       }
     }
-    if constexpr (kStates) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.hs) + b * T, p0, T, lane, Hk, wb, streamed);
+    if constexpr (kStates) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.hs) + b * T, p0, T, lane, Hk, wb);
     if constexpr (MODE == kSsGrad && kRound) {
-      if (a.gA_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SC *>(a.gA_step) + b * T, p0, T, lane, GA, wb, streamed);
-      if (a.gb_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.gb_step) + b * T, p0, T, lane, GB, wb, streamed);
-      if (a.gc_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.gc_step) + b * T, p0, T, lane, GC, wb, streamed);
-      if (a.gd_step) lpv_store_round<REV, kNVb>(a.gd_step + b * T, p0, T, lane, GD, wb, streamed);
+      if (a.gA_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SC *>(a.gA_step) + b * T, p0, T, lane, GA, wb);
+      if (a.gb_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.gb_step) + b * T, p0, T, lane, GB, wb);
+      if (a.gc_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.gc_step) + b * T, p0, T, lane, GC, wb);
+      if (a.gd_step) lpv_store_round<REV, kNVb>(a.gd_step + b * T, p0, T, lane, GD, wb);
     }
     if constexpr (MODE == kSsPlain || MODE == kSsStatesY)
-      lpv_store_round<REV, kNVb>(a.y + b * T, p0, T, lane, O, wb, streamed);
+      lpv_store_round<REV, kNVb>(a.y + b * T, p0, T, lane, O, wb);
     else if (MODE == kSsGrad && a.y)
-      lpv_store_round<REV, kNVb>(a.y + b * T, p0, T, lane, O, wb, streamed);
+      lpv_store_round<REV, kNVb>(a.y + b * T, p0, T, lane, O, wb);
   }
   if constexpr (MODE == kSsGrad) {
     if (a.gpart) {  // the wave's sums of the operands constant in time

@@ -123,7 +123,6 @@ struct ScanArgs {
   unsigned per_stripe;         // claims per stripe (grid = per_stripe * kStripes)
   unsigned spin_limit;         // look-back polls before the self-compute fallback
   unsigned agg_only;           // testing: tiles after a row's first publish no inclusive state
-  bool streamed;               // outputs leave past the caches (streams_out)
   // tile id -> (scan position, row) without a 64-bit division: for ids
   // below 2^31, id / B == (id * b_magic) >> b_shift (set by the host)
   uint64_t b_magic;
@@ -263,33 +262,15 @@ struct __attribute__((packed, aligned(4))) RowVec {
 };
 __device__ __forceinline__ RowVec row_vec(const uint4 &v) { return {v.x, v.y, v.z, v.w}; }
 
-// Stores past the caches.  The scans write every output once and are bound
-// by memory; a plain store's line stays in an L2 until it is written back
-// (at the latest as the launch ends) and takes the place of lines another
-// launch could read.  Kernel time, forward + backward, plain / streamed (us),
-// 16 fp32 rows: scalar scan of 131072 steps 19.6 / 18.0, 524288 58.8 / 56.6,
-// 2097152 232 / 220; 2x2 scan of 32768 23.7 / 22.5, 262144 100.4 / 93.3; the
-// time-varying biquad of 16384 23.2 / 23.4, 65536 39.4 / 37.0, 262144
-// 141.6 / 132.  With 8-byte elements the forward gains and a backward that
-// finds y in the 256 MB last-level cache may lose more: 64 fp64 rows of 32768
-// 27.8 / 28.5, 64 complex64 LTI rows of 32768 32.9 / 30.6, 65536
-// 45.8 / 46.2, 98304 65.8 / 61.1, 131072 86.6 / 88.0, 196608 124 / 126.3; from
-// 128 MB of outputs on, which with their inputs fill that cache, it only
-// gains: 262144 172 / 167.6, 524288 325 / 309.  So fp32 elements always
-// stream and wider ones from 128 MB on (streams_out in the launch code).
-// Kernels whose outputs the same call reads next (the cascades, filtfilt:
-// 40.7 / 43.1) store plainly.
-template <typename E>
-constexpr bool kStreamAlways = std::is_same<E, float>::value;
-
-// The empty statements keep this store and a plain one on the two sides of a
-// branch apart: merged, they lose the mark.
+// Stores past the caches: what a launch writes goes to memory at once instead
+// of holding L2 lines until the launch ends.  Worth it only where the outputs
+// are several times the 256 MB last-level cache and every store instruction
+// covers whole lines (scan_kernel's STREAM instantiations; kStreams here and
+// streams_out in the launch code say which launches).
 __device__ __forceinline__ void store_streamed(RowVec *p, const RowVec &v) {
   typedef uint32_t Words __attribute__((ext_vector_type(4), aligned(4)));
   const Words t = {v.x, v.y, v.z, v.w};
-  asm volatile("");
   __builtin_nontemporal_store(t, reinterpret_cast<Words *>(p));
-  asm volatile("");
 }
 
 // ------------------------------------------------------------ coalesced stores
@@ -330,8 +311,8 @@ __device__ __forceinline__ void lds_put_chunk(uint4 *wb, int L, const X (&v)[K])
 
 // The wave's buffer to its block at dst (in range): vector c of the block is
 // block lane c / NV's vector c % NV.
-template <int NV>
-__device__ __forceinline__ void lds_flush(void *dst, const uint4 *wb, int lane, bool write, bool streamed = false) {
+template <int NV, bool STREAM = false>
+__device__ __forceinline__ void lds_flush(void *dst, const uint4 *wb, int lane, bool write) {
   wave_sync();
   if (write) {
     RowVec *out = static_cast<RowVec *>(dst);
@@ -339,7 +320,7 @@ __device__ __forceinline__ void lds_flush(void *dst, const uint4 *wb, int lane, 
     for (int j = 0; j < NV; ++j) {
       const int c = j * 64 + lane, L = c / NV, v = c % NV;
       const RowVec u = row_vec(wb[L * NV + (v ^ lds_swizzle<NV>(L))]);
-      if (streamed)
+      if constexpr (STREAM)
         store_streamed(out + c, u);
       else
         out[c] = u;
@@ -501,9 +482,8 @@ __device__ __forceinline__ void load_chunk(const X *row, int64_t t0, int64_t T, 
   }
 }
 
-template <typename X, int K, bool kFull = false>
-__device__ __forceinline__ void store_chunk(X *row, int64_t t0, int64_t T, const X (&v)[K],
-                                            bool streamed = false) {
+template <typename X, int K, bool kFull = false, bool STREAM = false>
+__device__ __forceinline__ void store_chunk(X *row, int64_t t0, int64_t T, const X (&v)[K]) {
   if (kFull || t0 + K <= T) {
     constexpr int nv = int(K * sizeof(X) / 16);
     union {
@@ -515,7 +495,7 @@ __device__ __forceinline__ void store_chunk(X *row, int64_t t0, int64_t T, const
     RowVec *p = reinterpret_cast<RowVec *>(row + t0);
 #pragma unroll
     for (int i = 0; i < nv; ++i) {
-      if (streamed)
+      if constexpr (STREAM)
         store_streamed(p + i, u.v[i]);
       else
         p[i] = u.v[i];
@@ -638,6 +618,32 @@ __device__ __forceinline__ typename Alg::state tile_entry(const ScanArgs<Alg> &a
   return yin;
 }
 
+// Scans with a STREAM instantiation: the algebras and directions that gained,
+// all of whose stores cover whole lines (one vector a lane, or through LDS).
+// A lane's several vectors of its own, stored past the caches, reach memory
+// as partial lines: the 3x3 backward of 256 rows of 16384 steps took 401 us
+// for 106 (fp32) and 1100 for 195 (fp64).  The LTI forward does not gain (one
+// launch, plain / streamed: complex64, 1024 rows of 131072 steps 401 / 417 us,
+// fp64 404 / 406).
+template <class Alg>
+inline constexpr bool kStreamAlg = false;
+template <>
+inline constexpr bool kStreamAlg<Scalar<float>> = true;
+template <>
+inline constexpr bool kStreamAlg<Scalar<double>> = true;
+template <>
+inline constexpr bool kStreamAlg<Scalar<c64>> = true;
+template <>
+inline constexpr bool kStreamAlg<Block2<float>> = true;
+template <>
+inline constexpr bool kStreamAlg<Block2<double>> = true;
+template <typename X, int K>
+constexpr bool kWholeStores = K * int(sizeof(X)) == 16 || kLdsBlocked<X, K>;
+template <class Alg, bool TV, bool REV>
+constexpr bool kStreams = kStreamAlg<Alg> && (TV || REV) &&
+                          kWholeStores<typename Alg::s_state, Shape<Alg, TV>::K> &&
+                          (!(TV && REV) || kWholeStores<typename Alg::s_coef, Shape<Alg, TV>::K>);
+
 // ------------------------------------------------------------ the kernel
 // TV  : the coefficient varies along time (LPV); otherwise one per row (LTI).
 // REV : backward adjoint scan, nu[t] = A[t]^H (g[t] + nu[t+1]), run from the
@@ -674,7 +680,8 @@ __device__ __forceinline__ typename Alg::state tile_entry(const ScanArgs<Alg> &a
 //
 // TRACE: the instantiation a tracing launch runs; it also writes each
 // tile's phase record (kTraceWords words at trace + id * kTraceWords).
-template <class Alg, bool TV, bool REV, bool TRACE = false>
+// STREAM: the instantiation of launches whose outputs leave past the caches.
+template <class Alg, bool TV, bool REV, bool TRACE = false, bool STREAM = false>
 __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) void scan_kernel(ScanArgs<Alg> a) {
   using S = typename Alg::state;     // compute type
   using SC = typename Alg::s_coef;   // storage types
@@ -865,7 +872,6 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
       const int64_t blk0 = t0 - int64_t(pl) * K;
       const bool blk_full = kFull || blk0 + 64 * K <= T;
       uint4 *wb = s_out + w * 64 * kNVb;
-      const bool streamed = kStreamAlways<typename Alg::elem> || a.streamed;
       if constexpr (!REV) {
         SS O[K];
 #pragma unroll
@@ -876,10 +882,10 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
         if (kSLds && blk_full) {
           if constexpr (kSLds) {
             lds_put_chunk<SS, K>(wb, pl, O);
-            lds_flush<kNVs>(yrow + blk0, wb, lane, true, streamed);
+            lds_flush<kNVs, STREAM>(yrow + blk0, wb, lane, true);
           }
         } else {
-          store_chunk<SS, K, kFull>(yrow, t0, T, O, streamed);
+          store_chunk<SS, K, kFull, STREAM>(yrow, t0, T, O);
         }
       } else {
         SS nu = h;
@@ -902,19 +908,19 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
         if (kSLds && blk_full) {
           if constexpr (kSLds) {
             lds_put_chunk<SS, K>(wb, pl, GX);
-            lds_flush<kNVs>(gxrow + blk0, wb, lane, gxrow != nullptr, streamed);
+            lds_flush<kNVs, STREAM>(gxrow + blk0, wb, lane, gxrow != nullptr);
           }
         } else if (gxrow) {
-          store_chunk<SS, K, kFull>(gxrow, t0, T, GX, streamed);
+          store_chunk<SS, K, kFull, STREAM>(gxrow, t0, T, GX);
         }
         if constexpr (TV) {
           if (kCLds && blk_full) {
             if constexpr (kCLds) {
               lds_put_chunk<SC, K>(wb, pl, GC);
-              lds_flush<kNVc>(gcrow + blk0, wb, lane, gcrow != nullptr, streamed);
+              lds_flush<kNVc, STREAM>(gcrow + blk0, wb, lane, gcrow != nullptr);
             }
           } else if (gcrow) {
-            store_chunk<SC, K, kFull>(gcrow, t0, T, GC, streamed);
+            store_chunk<SC, K, kFull, STREAM>(gcrow, t0, T, GC);
           }
         }
       }
