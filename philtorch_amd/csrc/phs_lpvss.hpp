@@ -331,11 +331,18 @@ __device__ __noinline__ typename Alg::state lpv_prefix_fallback(const LpvSsArgs<
   return apply<Alg>(acc, virt);
 }
 
+// Waves per SIMD of the launch bounds: orders 1-2 hold 100 to 126 VGPRs in
+// every mode but the gradients' and run 4 (128 VGPRs; their fp32 instances,
+// unbounded, took 130 to 150 and lost one).
+template <class Alg, int MODE>
+constexpr int kLpvMinWaves = MODE != kSsGrad && SsView<Alg>::M <= 2 ? 4 : 2;
+
 // REV runs the model backwards in time: scan position s is time T-1-s (zi
 // the state before the last sample, zf after the first), the form of the
 // adjoint pass.  MODE as ss_kernel's.
 template <class Alg, bool REV, int MODE>
-__global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(LpvSsArgs<Alg> a) {
+__global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, (kLpvMinWaves<Alg, MODE>)) void lpv_ss_kernel(
+    LpvSsArgs<Alg> a) {
   using E = typename Alg::elem;
   using S = typename Alg::state;
   using SC = typename Alg::s_coef;
@@ -439,12 +446,19 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
     carry = compose<Alg>(carry, tot);
   }
   if (lane == 0) s_wagg[w] = carry;
-  // what pass 2 reads besides: orders 1-2 issue it before the wait for the
-  // entry state; orders 3-4, with no registers to hold it, step by step
+  // What pass 2 reads besides.  The gradient mode of orders 1-2 issues it
+  // before the wait for the entry state, and so do the other modes where four
+  // waves a SIMD have the registers to hold c and d (kPre); else they are
+  // read step by step, after it.  16 rows of 480000 steps, read before / step
+  // by step (us): order 1 fp32 44.8 / 49.2, order 2 fp64 218 / 226.  Order 2
+  // fp32 held them at three waves: 32 rows of 2^20 steps, forward 329 / 295,
+  // without c and d (held all the same) 287 / 239, with its states 366 / 325,
+  // with the x-only backward 597 / 509.
   const E *cp = a.cv.p ? a.cv.p + b * a.cv.row_stride : nullptr;
   const E *dp = a.d.p ? a.d.p + b * a.d.row_stride : nullptr;
   const SS c_fixed = V::unit(a.out_idx);
-  constexpr int kRe = kRound ? R : 1, kKe = kRound ? K : 1;
+  constexpr bool kPre = kRound && (MODE == kSsGrad || V::M == 1 || sizeof(E) == 8);
+  constexpr int kRe = kPre ? R : 1, kKe = kPre ? K : 1;
   SS Cv[kRe][kKe], Hf[MODE == kSsGrad ? R : 1][MODE == kSsGrad ? K : 1];
   E Dv[kRe][kKe], Xf[MODE == kSsGrad ? R : 1][MODE == kSsGrad ? K : 1];
   auto read_fwd = [&](int r) {
@@ -457,7 +471,7 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       read_fwd(r);
-      if constexpr (MODE != kSsStates) {
+      if constexpr (MODE != kSsStates && kPre) {
         if (cp) {
           lpv_operand<REV, SS, K>(a.cv, b, chunk0(r), T, Cv[r]);
         } else {
@@ -501,7 +515,7 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, 2) void lpv_ss_kernel(Lp
       if constexpr (MODE != kSsStates) {
         SS c;
         E dv;
-        if constexpr (kRound) {
+        if constexpr (kPre) {
           c = Cv[r][k];
           dv = Dv[r][k];
         } else {
