@@ -9,10 +9,16 @@
 namespace phs {
 namespace {
 
+template <class Alg, int F>
+constexpr int64_t mimo_least_tile() {
+  return MimoShape<Alg, F, MimoShape<Alg, F>::kHasShort>::kTile;
+}
 template <class Alg>
 size_t mimo_ws_bytes(int64_t B, int64_t T) {
-  // the shortest tile of any input width
-  constexpr int64_t tile = std::min<int64_t>(MimoShape<Alg, 1>::kTile, MimoShape<Alg, kMimoMaxIO>::kTile);
+  // the call does not say its input width: the shortest tile of any
+  constexpr int64_t t12 = std::min(MimoShape<Alg, 1>::kTile, MimoShape<Alg, 2>::kTile);
+  constexpr int64_t t34 = std::min(mimo_least_tile<Alg, 3>(), mimo_least_tile<Alg, 4>());
+  constexpr int64_t tile = std::min(t12, t34);
   const int64_t tiles = (T + tile - 1) / tile;
   return align_up(align_up(kHeaderBytes) + size_t(B) * size_t(tiles) * SsStatus<Alg>::kStride * sizeof(uint64_t));
 }
@@ -27,12 +33,12 @@ __global__ __launch_bounds__(256) void mimo_empty_zf_kernel(const E *zi, int64_t
   if (i < n) zf[i] = zi ? zi[i] : E(0);
 }
 
-template <class Alg, int F>
+template <class Alg, int F, bool SHORT>
 int mimo_ss_f(int P, int64_t B, int64_t T, const void *A, const void *Bm, const void *Cm, const void *Dm, int shared,
               const void *zi, const void *x, void *y, void *zf, void *workspace, size_t ws_bytes, bool rev,
               hipStream_t stream, void *hs) {
   using E = typename Alg::elem;
-  using Sh = MimoShape<Alg, F>;
+  using Sh = MimoShape<Alg, F, SHORT>;
   constexpr int M = SsView<Alg>::M;
   if (B < 0 || T < 0 || P < (hs ? 0 : 1) || P > kMimoMaxIO) return PHS_ERR_INVALID;
   if (shared & ~(PHS_MIMO_A_SHARED | PHS_MIMO_B_SHARED | PHS_MIMO_C_SHARED | PHS_MIMO_D_SHARED))
@@ -84,13 +90,13 @@ int mimo_ss_f(int P, int64_t B, int64_t T, const void *A, const void *Bm, const 
   const unsigned lds = unsigned(Sh::lds_bytes(P, hs != nullptr));
   if (hs) {
     if (rev)
-      launch_kernel((mimo_ss_kernel<Alg, F, true, true>), grid, block, lds, stream, a);
+      launch_kernel((mimo_ss_kernel<Alg, F, true, true, SHORT>), grid, block, lds, stream, a);
     else
-      launch_kernel((mimo_ss_kernel<Alg, F, false, true>), grid, block, lds, stream, a);
+      launch_kernel((mimo_ss_kernel<Alg, F, false, true, SHORT>), grid, block, lds, stream, a);
   } else if (rev) {
-    launch_kernel((mimo_ss_kernel<Alg, F, true, false>), grid, block, lds, stream, a);
+    launch_kernel((mimo_ss_kernel<Alg, F, true, false, SHORT>), grid, block, lds, stream, a);
   } else {
-    launch_kernel((mimo_ss_kernel<Alg, F, false, false>), grid, block, lds, stream, a);
+    launch_kernel((mimo_ss_kernel<Alg, F, false, false, SHORT>), grid, block, lds, stream, a);
   }
   return hipGetLastError() == hipSuccess ? PHS_OK : PHS_ERR_LAUNCH;
 }
@@ -100,8 +106,15 @@ int mimo_ss(int F, int P, int64_t B, int64_t T, const void *A, const void *Bm, c
             int shared, const void *zi, const void *x, void *y, void *zf, void *workspace, size_t ws_bytes, bool rev,
             hipStream_t stream, void *hs = nullptr) {
   auto run = [&](auto f) {
-    return mimo_ss_f<Alg, decltype(f)::value>(P, B, T, A, Bm, Cm, Dm, shared, zi, x, y, zf, workspace, ws_bytes, rev,
-                                              stream, hs);
+    constexpr int Fc = decltype(f)::value;
+    using Sh = MimoShape<Alg, Fc>;
+    if constexpr (Sh::kHasShort) {
+      if (B > 0 && T > 0 && double(B) * double((T + Sh::kTile - 1) / Sh::kTile) < double(kMimoShortTiles))
+        return mimo_ss_f<Alg, Fc, true>(P, B, T, A, Bm, Cm, Dm, shared, zi, x, y, zf, workspace, ws_bytes, rev,
+                                        stream, hs);
+    }
+    return mimo_ss_f<Alg, Fc, false>(P, B, T, A, Bm, Cm, Dm, shared, zi, x, y, zf, workspace, ws_bytes, rev, stream,
+                                     hs);
   };
   switch (F) {
     case 1: return run(std::integral_constant<int, 1>{});

@@ -23,8 +23,10 @@
 // (lpv_mimo_kernel) stages its inputs through such planes too.  The
 // reversed mode (REV) runs the model backwards in time: the gradients w.r.t.
 // x and zi are that mode on the adjoint model (A^T, input matrix C^T, output
-// matrix B^T, feedthrough D^T); with C = I and no D the output is the state
-// before every step, which the coefficient gradients reduce against.
+// matrix B^T, feedthrough D^T).  The coefficient gradients reduce against the
+// state before every step, which the LTI kernel's HS mode writes beside the
+// outputs or alone, and the time-varying kernel gives where P + M fit its
+// planes, else as its output with C = I and no D.
 #pragma once
 
 #include "phs_lpvss.hpp"
@@ -81,13 +83,21 @@ struct MimoArgs {
 // model in scalar registers and 16 steps a lane 58 (2.1 TB/s).  8 steps a
 // lane take 76, 7 data waves 76; 3 in and 3 out 115 -> 74 (8 steps: 85);
 // order 2, 1 in and 1 out 56 -> 31; order 4 fp64 (16 x 240000) 115 -> 60.
-template <class Alg, int F>
+//
+// Half as many steps a lane where 64 bytes of every feature are too many:
+// order 4 with 4 inputs in fp32 always (4 out: with 16 steps a lane it
+// spilled 46 to 66 VGPRs and took 125 us for 107, 16 x 24001 27.1 for 21.3),
+// and in fp64 with 3 or 4 inputs in the SHORT form, for launches whose tiles
+// would not fill the chip (kMimoShortTiles).
+template <class Alg, int F, bool SHORT = false>
 struct MimoShape {
   using E = typename Alg::elem;
   static constexpr int M = int(sizeof(typename Alg::s_state) / sizeof(E));
+  static constexpr bool kHasShort = sizeof(E) == 8 && M == 4 && F >= 3;
+  static_assert(kHasShort || !SHORT, "no short form");
   static constexpr int kWaves = 3;
   static constexpr int kThreads = 64 * (kWaves + 1);
-  static constexpr int K = 64 / int(sizeof(E));
+  static constexpr int K = (SHORT || (sizeof(E) == 4 && M == 4 && F == 4) ? 32 : 64) / int(sizeof(E));
   static constexpr int kSpan = 64 * K;
   static constexpr int kTile = kWaves * kSpan;
   static constexpr int kPitch = K + 1;
@@ -103,6 +113,13 @@ struct MimoShape {
   }
   static constexpr __host__ __device__ size_t align16(size_t n) { return (n + 15) / 16 * 16; }
 };
+
+// Fewer tiles than this take the SHORT form: two workgroups of the long one
+// fit a CU.  Order 4 fp64, 4 in and 4 out, forward (us), long / short: 16 x
+// 3000 24.8 / 18.1, 16 x 24001 (256 long tiles) 28.1 / 23.6, 16 x 131072
+// (1376) 76.0 / 78.0, 1024 x 4096 (3072) 129 / 139; 3 in and 4 out 21.4 /
+// 17.4, 23.8 / 21.6, 63.7 / 72.6, 108 / 132.
+constexpr int64_t kMimoShortTiles = 512;
 
 // The span's element e of a [T, P] row block: step e / P, output e % P, for
 // e < 64 K P <= 4096 (24-bit multiplies; magic = ceil(2^18 / P)).
@@ -408,13 +425,13 @@ __device__ __forceinline__ typename Alg::state mimo_lane_fold(const MimoModel<Al
 // State entering tile position `span` of a row, folded from the inputs (the
 // look-back's bounded-wait fallback; out of line, cold): 64 K steps at a
 // time, st <- A^(64 K) st + the chunk's total.
-template <class Alg, int F, bool REV>
+template <class Alg, int F, bool REV, bool SHORT>
 __device__ __noinline__ typename Alg::state mimo_prefix_fallback(const MimoArgs<Alg> *ap, int64_t b, int64_t span,
                                                                 int lane, typename Alg::state st,
                                                                 const SsPowers<Alg> *tab) {
   const MimoArgs<Alg> &a = *ap;
   using X = IoVec<typename Alg::elem, F>;
-  constexpr int K = MimoShape<Alg, F>::K;
+  constexpr int K = MimoShape<Alg, F, SHORT>::K;
   MimoModel<Alg, F> m;
   mimo_model<Alg, F>(a, b, m);
   const X *xrow = reinterpret_cast<const X *>(a.x) + b * a.T_len;
@@ -432,14 +449,14 @@ __device__ __noinline__ typename Alg::state mimo_prefix_fallback(const MimoArgs<
 // HS: also the state before every step into a.hs (with P = 0 the states
 // alone): 16 x 480000 fp32, order 4, 2 in 2 out, 76 us with the outputs and 62
 // without, where a second pass with C the identity took 95.
-template <class Alg, int F, bool REV, bool HS>
-__global__ __launch_bounds__((MimoShape<Alg, F>::kThreads), (MimoShape<Alg, F>::kMinWaves)) void mimo_ss_kernel(
-    MimoArgs<Alg> a) {
+template <class Alg, int F, bool REV, bool HS, bool SHORT>
+__global__ __launch_bounds__((MimoShape<Alg, F, SHORT>::kThreads),
+                             (MimoShape<Alg, F, SHORT>::kMinWaves)) void mimo_ss_kernel(MimoArgs<Alg> a) {
   using E = typename Alg::elem;
   using S = typename Alg::state;
   using SS = typename Alg::s_state;
   using V = SsView<Alg>;
-  using Sh = MimoShape<Alg, F>;
+  using Sh = MimoShape<Alg, F, SHORT>;
   using St = SsStatus<Alg>;
   using X = IoVec<E, F>;
   constexpr int K = Sh::K, kWaves = Sh::kWaves, kP = Sh::kPlane, M = V::M;
@@ -488,7 +505,7 @@ __global__ __launch_bounds__((MimoShape<Alg, F>::kThreads), (MimoShape<Alg, F>::
     if (q > 0) {
       if (lane == 0) publish(row_status + q * St::kStride + St::kVecWords, tagg, tag);
       if (!ss_lookback<Alg>(row_status, virt, lane, tag, a.spin_limit, s_look, &s_tab, q, yin))
-        yin = mimo_prefix_fallback<Alg, F, REV>(kernel_args<MimoArgs<Alg>>(), b, q * Sh::kTile, lane, virt, &s_tab);
+        yin = mimo_prefix_fallback<Alg, F, REV, SHORT>(kernel_args<MimoArgs<Alg>>(), b, q * Sh::kTile, lane, virt, &s_tab);
     }
     if (q + 1 < a.tiles_per_row && lane == 0 && !(a.agg_only && q > 0))
       publish(row_status + q * St::kStride, Alg::affine(s_tab.gp[0], yin, tagg), tag);
