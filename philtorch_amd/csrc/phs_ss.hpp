@@ -131,7 +131,6 @@ struct SsShape {
   static constexpr int M = int(sizeof(typename Alg::s_state) / sizeof(E));
   static constexpr bool kWide = MODE == kSsPlain && M == 2 && sizeof(E) == 4;
   static constexpr int kWaves = kWide ? 15 : 3;
-  static constexpr int kMinWaves = kWide ? 4 : 2;  // waves per SIMD the launch bounds ask for
   static constexpr int kThreads = 64 * (kWaves + 1);
   static constexpr int K = kWide ? 16 : int((M <= 2 ? 32 : 64) / sizeof(E));
   static constexpr int R = kWide ? 2 : (M <= 2 ? 4 : 2) / (MODE == kSsGrad ? 2 : 1);
@@ -145,6 +144,19 @@ struct SsShape {
   static constexpr int kLdsRounds = kWide ? 1 : 0;
   static_assert((K & (K - 1)) == 0, "K is a power of two (the lane matrix is A^K by squaring)");
 };
+
+// Waves per SIMD the launch bounds ask for.  Order 1 fp64 fits 96 VGPRs (five
+// waves) but takes 98 unasked: lfilter of 16 x 480000 steps, four / five
+// waves, 36.0 / 33.9 us, of 24 x 300000 35.2 / 32.7.  Its reversed plain pass
+// spills there and short rows lose (16 x 3000 with the x gradient 13.9 /
+// 14.7); order 1 fp32 spills in most modes and gains at some sizes what it
+// loses at others.
+template <class Alg, bool REV, int MODE>
+constexpr int kSsMinWaves = SsShape<Alg, MODE>::kWide ? 4
+                            : SsShape<Alg, MODE>::M == 1 && sizeof(typename Alg::elem) == 8 &&
+                                    (MODE == kSsStatesY || (MODE == kSsPlain && !REV))
+                                ? 5
+                                : 2;
 
 // Chunk I/O in scan order: forward, scan position s is time s; reversed
 // (REV), it is time T-1-s, so a lane's K steps are the K samples below
@@ -834,7 +846,7 @@ __device__ __forceinline__ void issue_barrier() {
 }
 
 template <class Alg, bool REV, int MODE>
-__global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (SsShape<Alg, MODE>::kMinWaves)) void ss_kernel(
+__global__ __launch_bounds__((SsShape<Alg, MODE>::kThreads), (kSsMinWaves<Alg, REV, MODE>)) void ss_kernel(
     SsArgs<Alg> a) {
   using E = typename Alg::elem;
   using S = typename Alg::state;
