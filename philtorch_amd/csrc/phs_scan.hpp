@@ -246,6 +246,21 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// v's value from here on is not known to the compiler: nothing computed from
+// it later moves above this point.
+template <typename X>
+__device__ __forceinline__ void keep_here(X &v) {
+  static_assert(sizeof(X) % 4 == 0, "whole registers");
+  union {
+    X x;
+    uint32_t w[sizeof(X) / 4];
+  } u;
+  u.x = v;
+#pragma unroll
+  for (int i = 0; i < int(sizeof(X) / 4); ++i) asm volatile("" : "+v"(u.w[i]));
+  v = u.x;
+}
+
 // ------------------------------------------------------------ vectors of a row
 // Rows are read and written 16 bytes at a time wherever the 16 bytes lie
 // inside them, at any element alignment: a global memory instruction of four
@@ -860,6 +875,13 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
       }
     }
 
+    // LTI: the row's coefficient, opaque from here.  Left to itself the
+    // compiler moves what both forms of the path compute from it ahead of the
+    // branch between them, where it waits for the coefficient, and for the
+    // claim issued before it, ahead of the tile's loads.
+    SC a_row = a_row_s;
+    if constexpr (!TV && kOwnClaim) keep_here(a_row);
+
     // ---- pass 2 of round r from the start state h, writing its outputs
     // backward: y[t0-1] of each round sits in the last step of the next
     // lane's chunk (lanes are mirrored), or below the round for lane 63 (set,
@@ -876,7 +898,7 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
         SS O[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-          h = Alg::s_affine(TV ? A[r][TV ? k : 0] : a_row_s, h, X[r][k]);
+          h = Alg::s_affine(TV ? A[r][TV ? k : 0] : a_row, h, X[r][k]);
           O[k] = h;
         }
         if (kSLds && blk_full) {
@@ -894,7 +916,7 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
           const int k = K - 1 - kk;
-          const SC c = Alg::s_adjoint(TV ? A[r][TV ? k : 0] : a_row_s);
+          const SC c = Alg::s_adjoint(TV ? A[r][TV ? k : 0] : a_row);
           const SS lam = Alg::s_add(X[r][k], nu);
           GX[k] = lam;
           const SC g = Alg::s_outer(lam, k == 0 ? Ybelow[r] : Y[r][k > 0 ? k - 1 : 0]);
@@ -933,7 +955,7 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
     M carry = map_identity<Alg>();
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      M m = lane_map<Alg, TV, REV, K>(A[TV ? r : 0], X[r], a_row_s);
+      M m = lane_map<Alg, TV, REV, K>(A[TV ? r : 0], X[r], a_row);
       m = wave_scan_incl(m, lane, op);
       const M ex = wave_shift_up(m, lane, map_identity<Alg>());
       const M tot = read_lane(m, 63);
