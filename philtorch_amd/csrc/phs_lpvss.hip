@@ -55,8 +55,17 @@ LpvSsArgs<Alg> lpv_args(int64_t B, int64_t T, const void *A, bool A_sh, bool A_t
   return a;
 }
 
+constexpr double kLpvStreamedBytes = 16777216.0;
+
 template <class Alg, bool REV, int MODE = kSsPlain>
-int lpv_launch(const LpvSsArgs<Alg> &a, hipStream_t stream) {
+int lpv_launch(const LpvSsArgs<Alg> &a, hipStream_t stream, bool stream_out = false) {
+  if constexpr (kLpvStreams<Alg, MODE>) {
+    if (stream_out) {
+      launch_kernel((lpv_ss_kernel<Alg, REV, MODE, true>), dim3(a.per_stripe * kStripes),
+                    dim3(LpvSsShape<Alg>::kThreads), 0, stream, a);
+      return hipGetLastError() == hipSuccess ? PHS_OK : PHS_ERR_LAUNCH;
+    }
+  }
   launch_kernel((lpv_ss_kernel<Alg, REV, MODE>), dim3(a.per_stripe * kStripes), dim3(LpvSsShape<Alg>::kThreads), 0,
                 stream, a);
   return hipGetLastError() == hipSuccess ? PHS_OK : PHS_ERR_LAUNCH;
@@ -190,7 +199,17 @@ int lpv_ss_bwd(int64_t B, int64_t T, const void *A, bool A_sh, bool A_tr, LpvOpe
     q.gA_trans = A_tr ? 1 : 0;
     q.sum_b = sum_b, q.sum_c = sum_c, q.sum_d = sum_d;
     q.gpart = (sum_b || sum_c || sum_d) ? gpart : nullptr;
-    rc = rev ? lpv_launch<Alg, false, kSsGrad>(q, stream) : lpv_launch<Alg, true, kSsGrad>(q, stream);
+    // past the caches from 16 MiB of outputs on (below, within 2 % either way),
+    // unless the batch sums read some of them next
+    const int64_t width[4] = {M * M, M, M, 1};
+    int64_t per_step = gx ? 1 : 0;
+    bool read_next = false;
+    for (int i = 0; i < 4; ++i) {
+      if (step_dst[i]) per_step += width[i];
+      read_next |= step_dst[i] && step_dst[i] != outs[i];
+    }
+    const bool so = !read_next && double(B) * double(T) * double(per_step) * double(sizeof(E)) >= kLpvStreamedBytes;
+    rc = rev ? lpv_launch<Alg, false, kSsGrad>(q, stream, so) : lpv_launch<Alg, true, kSsGrad>(q, stream, so);
     if (rc != PHS_OK) return rc;
   }
   // operands shared by the rows and varying along time: sums over the rows

@@ -125,12 +125,12 @@ __device__ __forceinline__ void lpv_load(const X *row, int64_t s0, int64_t T, X 
   }
 }
 
-template <bool REV, typename X, int K>
+template <bool REV, typename X, int K, bool STREAM = false>
 __device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X (&v)[K]) {
   constexpr bool kVec = (K * sizeof(X)) % 16 == 0;
   if constexpr (!REV) {
     if constexpr (kVec) {
-      store_chunk<X, K>(row, s0, T, v);
+      store_chunk<X, K, false, STREAM>(row, s0, T, v);
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k)
@@ -142,7 +142,7 @@ __device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X
       X tmp[K];
 #pragma unroll
       for (int k = 0; k < K; ++k) tmp[k] = v[K - 1 - k];
-      if constexpr (kVec) store_chunk<X, K>(row, base, T, tmp);
+      if constexpr (kVec) store_chunk<X, K, false, STREAM>(row, base, T, tmp);
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
@@ -164,8 +164,9 @@ __device__ __forceinline__ void lpv_store(X *row, int64_t s0, int64_t T, const X
 // row: where a lane's chunk is more than one 16-byte vector and the round
 // lies inside the row, through the wave's LDS buffer `wb` (lds_flush: 1 KB of
 // the row an instruction), else a lane's own vectors.
-// NB: the buffer's vectors a lane.
-template <bool REV, int NB, typename X, int K>
+// NB: the buffer's vectors a lane.  STREAM: past the caches, which a lane's own
+// vectors are only where it has one (kWholeStores).
+template <bool REV, int NB, bool STREAM, typename X, int K>
 __device__ __forceinline__ void lpv_store_round(X *row, int64_t p0, int64_t T, int lane, const X (&v)[K], uint4 *wb) {
   if constexpr (kLdsBlocked<X, K>) {
     static_assert(K * int(sizeof(X)) / 16 <= NB, "the round fits the wave's buffer");
@@ -179,11 +180,11 @@ __device__ __forceinline__ void lpv_store_round(X *row, int64_t p0, int64_t T, i
       } else {
         lds_put_chunk<X, K>(wb, lane, v);
       }
-      lds_flush<NV>(row + (REV ? T - p0 - 64 * K : p0), wb, lane, true);
+      lds_flush<NV, STREAM>(row + (REV ? T - p0 - 64 * K : p0), wb, lane, true);
       return;
     }
   }
-  lpv_store<REV, X, K>(row, p0 + int64_t(lane) * K, T, v);
+  lpv_store<REV, X, K, STREAM && K * int(sizeof(X)) == 16>(row, p0 + int64_t(lane) * K, T, v);
 }
 
 // Time of scan position s (clamped into the row: positions past it carry a
@@ -340,7 +341,19 @@ constexpr int kLpvMinWaves = MODE != kSsGrad && SsView<Alg>::M <= 2 ? 4 : 2;
 // REV runs the model backwards in time: scan position s is time T-1-s (zi
 // the state before the last sample, zf after the first), the form of the
 // adjoint pass.  MODE as ss_kernel's.
-template <class Alg, bool REV, int MODE>
+//
+// STREAM (kLpvStreams): the gradient mode's outputs leave past the caches, as
+// nothing of the same call reads them.  With every gradient, passes in turn
+// among others, plain / streamed (us): order 2 fp32, 16 x 441000 217.7 / 204.2,
+// 24 x 262145 194.8 / 176.0, 32 x 2^20 888 / 869, fp64 64 x 131072 544 / 532;
+// order 1 fp32, 64 x 262144 245.9 / 228.0.  With the operands evicted before
+// every pass: order 2 fp32, 1024 x 4096 119.5 / 111.9, 16 x 131072 78.0 /
+// 75.3, 16 x 441000 211.6 / 210.9; order 1 fp64, 16 x 441000 214.4 / 217.9,
+// 1024 x 4096 117.0 / 108.2.
+template <class Alg, int MODE>
+constexpr bool kLpvStreams = MODE == kSsGrad && SsView<Alg>::M <= 2;
+
+template <class Alg, bool REV, int MODE, bool STREAM = false>
 __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, (kLpvMinWaves<Alg, MODE>)) void lpv_ss_kernel(
     LpvSsArgs<Alg> a) {
   using E = typename Alg::elem;
@@ -549,17 +562,17 @@ __global__ __launch_bounds__(LpvSsShape<Alg>::kThreads, (kLpvMinWaves<Alg, MODE>
         for (int i = 0; i < V::M; ++i) a.zf[b * V::M + i] = zu.e[i];
       }
     }
-    if constexpr (kStates) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.hs) + b * T, p0, T, lane, Hk, wb);
+    if constexpr (kStates) lpv_store_round<REV, kNVb, STREAM>(reinterpret_cast<SS *>(a.hs) + b * T, p0, T, lane, Hk, wb);
     if constexpr (MODE == kSsGrad && kRound) {
-      if (a.gA_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SC *>(a.gA_step) + b * T, p0, T, lane, GA, wb);
-      if (a.gb_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.gb_step) + b * T, p0, T, lane, GB, wb);
-      if (a.gc_step) lpv_store_round<REV, kNVb>(reinterpret_cast<SS *>(a.gc_step) + b * T, p0, T, lane, GC, wb);
-      if (a.gd_step) lpv_store_round<REV, kNVb>(a.gd_step + b * T, p0, T, lane, GD, wb);
+      if (a.gA_step) lpv_store_round<REV, kNVb, STREAM>(reinterpret_cast<SC *>(a.gA_step) + b * T, p0, T, lane, GA, wb);
+      if (a.gb_step) lpv_store_round<REV, kNVb, STREAM>(reinterpret_cast<SS *>(a.gb_step) + b * T, p0, T, lane, GB, wb);
+      if (a.gc_step) lpv_store_round<REV, kNVb, STREAM>(reinterpret_cast<SS *>(a.gc_step) + b * T, p0, T, lane, GC, wb);
+      if (a.gd_step) lpv_store_round<REV, kNVb, STREAM>(a.gd_step + b * T, p0, T, lane, GD, wb);
     }
     if constexpr (MODE == kSsPlain || MODE == kSsStatesY)
-      lpv_store_round<REV, kNVb>(a.y + b * T, p0, T, lane, O, wb);
+      lpv_store_round<REV, kNVb, STREAM>(a.y + b * T, p0, T, lane, O, wb);
     else if (MODE == kSsGrad && a.y)
-      lpv_store_round<REV, kNVb>(a.y + b * T, p0, T, lane, O, wb);
+      lpv_store_round<REV, kNVb, STREAM>(a.y + b * T, p0, T, lane, O, wb);
   }
   if constexpr (MODE == kSsGrad) {
     if (a.gpart) {  // the wave's sums of the operands constant in time

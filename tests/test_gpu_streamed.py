@@ -99,6 +99,47 @@ def test_past_the_caches(hip, kind, T, rows):
             assert float((p[lo:hi] - q).abs().max()) <= tol * float(q.abs().max()), i
 
 
+# 16 MiB of per-step gradients and grad_x, from which on the time-varying state
+# space's gradients leave past the caches: just above, and halves below
+@pytest.mark.parametrize("T", [4096, 4099])
+@pytest.mark.parametrize("operands", ["every one", "shared A", "constant b"])
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("dt", ["float32", "float64"])
+def test_state_space_gradients(hip, dt, M, operands, T):
+    """One launch that streams against two of half its rows that do not.  With
+    A shared by the rows its gradient is a sum over them, of rows that each
+    agree as above: the halves' sums add up to the whole's."""
+    import torch
+
+    from philtorch_amd import lpv
+
+    dt = getattr(torch, dt)
+    es = torch.empty((), dtype=dt).element_size()
+    per_step = {"every one": M * M + M + 2, "shared A": M * M + M + 2, "constant b": M * M + 1}[operands] * es
+    B = 2 * (-(-(1 << 24) // (T * per_step)) // 2 + 1)
+    g = torch.Generator(device="cuda").manual_seed(B + T)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=dt)  # noqa: E731
+    A = ((torch.rand(*(() if operands == "shared A" else (B,)), T, M, M, generator=g, device="cuda") - 0.5) * 0.9).to(dt)
+    b, d = (r(M), None) if operands == "constant b" else (r(B, T, M), r(B, T))
+    zi, x, gy = r(B, M), r(B, T), r(B, T)
+
+    def run(lo, hi):
+        part = lambda t: t if t is None or t.size(0) != B else t[lo:hi].contiguous()  # noqa: E731
+        ts = [None if t is None else part(t).detach().requires_grad_(True) for t in (A, b, d, zi, x)]
+        y, zf = lpv.state_space(ts[0], ts[4], B=ts[1], D=ts[2], zi=ts[3], unroll_factor=1, out_idx=0)
+        wanted = [t for t in ts if t is not None]
+        return [y.detach(), zf.detach()] + list(torch.autograd.grad(y, wanted, gy[lo:hi].contiguous()))
+
+    whole, first, second = run(0, B), run(0, B // 2), run(B // 2, B)
+    eps = torch.finfo(dt).eps
+    for i, (w, p, q) in enumerate(zip(whole, first, second)):
+        if w.size(0) == B:
+            want, tol = torch.cat([p, q]), 64 * eps
+        else:  # summed over the rows
+            want, tol = p + q, 64 * eps * B ** 0.5
+        assert float((w - want).abs().max()) <= tol * float(want.abs().max()), i
+
+
 @pytest.mark.parametrize("dt", ["float32", "float64"])
 def test_3x3_backward_time(hip, dt):
     """The 3x3 scan's stores are a lane's own vectors, 36 to 144 bytes apart:

@@ -68,7 +68,7 @@ def test_time_varying_state_space_holds_four_waves(kernels):
     forward took 130 to 150 and ran 10 to 19 % slower at order 2.)"""
     for name, k in _some(kernels, r"lpv_ss_kernelINS_6(Scalar|Block2)I[fd]EELb[01]ELi[013]E"):
         assert k[".vgpr_count"] <= 128, (name, k[".vgpr_count"])
-        if "ELb0E" in name:
+        if "EELb0ELi" in name:  # forward in time
             assert k[".vgpr_spill_count"] == 0, name
 
 
@@ -94,3 +94,7 @@ def test_streaming_instantiations(kernels):
              for n, _ in _some(kernels, r"scan_kernelI.*ELb[01]ELb[01]ELb0ELb1E")}
     algs = {"6ScalarIf", "6ScalarId", "6ScalarINS_3c64E", "6Block2If", "6Block2Id"}
     assert names == {(a, tv, rev) for a in algs for tv, rev in (("1", "0"), ("1", "1"), ("0", "1"))}
+    # the time-varying state space: the gradient mode (2) of orders 1-2
+    modes = {re.search(r"lpv_ss_kernelINS_6(.*?)EELb.ELi(.)ELb1E", n).groups()
+             for n, _ in _some(kernels, r"lpv_ss_kernelI.*ELi.ELb1E")}
+    assert modes == {(a, "2") for a in ("ScalarIf", "ScalarId", "Block2If", "Block2Id")}
