@@ -659,6 +659,20 @@ constexpr bool kStreams = kStreamAlg<Alg> && (TV || REV) &&
                           kWholeStores<typename Alg::s_state, Shape<Alg, TV>::K> &&
                           (!(TV && REV) || kWholeStores<typename Alg::s_coef, Shape<Alg, TV>::K>);
 
+// The time-invariant 2x2 fp32 backward has every round's y in registers before
+// pass 2.  A wait counts loads and stores alike, so one for the second round's
+// y, between the rounds of pass 2, waits for the first round's stores as well;
+// the loads themselves have had the look-back's time.  Backward (us), with
+// waits between the rounds / without: 32 x 10^6 180.5 / 174.3, 64 x 500000
+// 180.1 / 171.9, 256 x 65536 99.3 / 95.4, 32 x 2^22 695 / 649, 16 x 480000 57.1
+// / 57.0, 1024 x 262144 1234 / 1239.  Complex64, the other with two rounds
+// through LDS, gains at some sizes what it loses at others (256 x 65536 91.6 /
+// 88.9, 1024 x 262144 1253 / 1274), and real scalars and order 3 nothing.
+template <class Alg, bool TV, bool REV>
+constexpr bool kYFirst = false;
+template <>
+inline constexpr bool kYFirst<Block2<float>, false, true> = true;
+
 // ------------------------------------------------------------ the kernel
 // TV  : the coefficient varies along time (LPV); otherwise one per row (LTI).
 // REV : backward adjoint scan, nu[t] = A[t]^H (g[t] + nu[t+1]), run from the
@@ -997,6 +1011,14 @@ __global__ __launch_bounds__((Shape<Alg, TV>::kThreads), Alg::kMinWavesPerEU) vo
     M wpre = map_identity<Alg>();
     for (int j = 0; j < w; ++j) wpre = compose<Alg>(wpre, s_wagg[j]);
     __syncthreads();  // entry state is in s_in
+
+    if constexpr (kYFirst<Alg, TV, REV>) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) keep_here(Y[r][k]);
+      }
+    }
 
     // ---- pass 2 from the entry state
     const S hin = apply<Alg>(wpre, s_in);  // state entering this wave's segment
